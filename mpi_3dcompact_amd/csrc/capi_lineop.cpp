@@ -23,7 +23,7 @@ struct mc3d_lineop {
     bool fast = false;      // plain applications use the fast kernels
     std::string kname;      // kernel of plain applications
     // transformed-periodic applications run the LDS-tiled kernel, which takes
-    // 16- and 32-row chunks only: a 16-row twin when the plain plan has others
+    // 16- and 32-row chunks only: a 16-row (or 32-row) twin when the plain plan has others
     mc3d_lineop *tpb = nullptr;
 };
 
@@ -162,6 +162,33 @@ int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
             return mc3d::fail(rc, err);
         }
     }
+    // Banded ragged lines of 512 lines or more, in 20-row chunks (28 where those
+    // leave the short chunk fewer than 2W rows) and one short chunk:
+    //  - lines whose remainder over 16 (32) rows is too short for its interface
+    //    blocks (65, 129, 193 points, say), which only the LDS-tiled kernel
+    //    took: 129-point Penta10 y in a 160 x 129 x 144 box, four fields,
+    //    305 -> 42 us (0.62 -> 4.6 TB/s; 28 rows 50 us), Compact8 138 -> 48;
+    //    193-point x 1450 -> 399 and 748 -> 351 us (three fields);
+    //  - y- and z-lines of 257 to 320 points, at most 16 chunks: 310-point
+    //    Penta10 z 231 -> 200 us against 32-row chunks (4.0 -> 4.6 TB/s), Compact8
+    //    210 -> 189 (28 rows 199).  Shorter ragged y- and z-lines keep 16 rows
+    //    (165 points: 67 against 70 us), longer ones 32.
+    // Fewer lines keep the plan's own choice: one field of so small a box is
+    // launch latency either way (272 Penta10 lines of 131 points 21 -> 11 us).
+    const bool banded = op->plan.W > 0 && !tune.mm && tune.family != 2;
+    const long nlines = npts / nbatch / dims[dir];  // one member's: a stacked box takes its members' kernels
+    const int planned = op->plan.MM;
+    const bool rescue = !op->fast, mid = op->fast && dir != 0 && op->plan.cshort >= 0 && op->plan.MM == 32 && dims[dir] <= 320;
+    if (banded && nlines >= 512 && (rescue || mid)) {
+        for (int mm : {20, 28}) {
+            if (dims[dir] % mm == 0 || (mid && mm == 28)) continue;
+            if (plan_with(mm) == MC3D_OK && op->fast) break;
+        }
+        if (!op->fast && (rc = plan_with(planned)) != MC3D_OK) {
+            delete op;
+            return mc3d::fail(rc, err);
+        }
+    }
     if (!op->fast && op->plan.MM != 16 && op->plan.MM != 32) {  // the LDS-tiled kernel's chunk sizes
         delete op;
         return mc3d::fail(MC3D_EINVAL, "no kernel for this line operator and chunking");
@@ -212,6 +239,10 @@ int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
         t.mm = 16;
         t.family = 2;
         rc = create(cls, kind, dir, bc, bc3, dims, dd, alphaF, nbatch, t, &op->tpb);
+        if (rc) {  // 305 points, say: 19 chunks of 16 rows and one of a single row
+            t.mm = 32;
+            rc = create(cls, kind, dir, bc, bc3, dims, dd, alphaF, nbatch, t, &op->tpb);
+        }
         if (rc) {
             mc3d_lineop_destroy(op);
             return rc;

@@ -82,9 +82,11 @@ bool lineop_fast_supported(const OpDev &op, size_t lds_limit) {
     const bool ends = op.periodic ? (op.nbl + op.nbr == 0 || (w == 0 && h == 1 && op.nbl == h && op.nbr == h))
                                   : (op.nbl == h && op.nbr == h);
     const bool rows = chunk_rows_ok(op.MM) && (op.MM >= 16 || op.periodic) && op.MM >= 2 * h;
-    // evenly chunked, or ragged: 16- or 32-row chunks and one short second chunk
+    // evenly chunked, or ragged: 16- or 32-row chunks (banded operators 20- and
+    // 28-row ones too) and one short second chunk
     const bool chunks = op.cshort < 0 ? op.N == op.P * op.MM
-                                      : (op.MM == 16 || op.MM == 32) && op.cshort == 1 && op.P >= 3 &&
+                                      : (op.MM == 16 || op.MM == 32 || (w > 0 && (op.MM == 20 || op.MM == 28))) &&
+                                            op.cshort == 1 && op.P >= 3 &&
                                             op.lshort >= std::max(2 * w, 1) && op.lshort < op.MM &&
                                             op.N == (op.P - 1) * op.MM + op.lshort;
     return pair && ends && rows && chunks && threads <= 1024 && lineop_fast_lds_bytes(op) <= lds_limit;

@@ -1153,7 +1153,7 @@ hipError_t launch_fast(const OpDev &op, const LaunchArgs &a, int nfields, hipStr
         }
         hipLaunchKernelGGL((lineop_contig<W, H, MM, PER, RG, L>), grid, block, lineop_fast_lds_bytes(op), st, op, a);
     } else {
-        if constexpr ((!RG && ((PER && !has_rows<W, H, PER>()) || MM == 16 || MM == 32)) || (RG && !PER)) {
+        if constexpr ((!RG && ((PER && !has_rows<W, H, PER>()) || MM == 16 || MM == 32)) || (RG && !PER && MM % 16 == 0)) {
             if (lineop_fast_pair(op)) {
                 dim3 grid((a.nlines + 31) / 32, nfields, op.dir == 2 ? a.nbatch : 1), block(64, lineop_pair_waves(op));
                 hipLaunchKernelGGL((lineop_strided_pair<W, H, MM, PER, RG>), grid, block, lineop_fast_lds_bytes(op),
@@ -1186,6 +1186,10 @@ hipError_t launch_fast_mm(const OpDev &op, const LaunchArgs &a, int nfields, hip
     if (op.cshort >= 0) {  // ragged lines: 16- or 32-row chunks and one short chunk
         if (op.MM == 16) return launch_fast_bc<W, H, 16, true>(op, a, nfields, st);
         if (op.MM == 32) return launch_fast_bc<W, H, 32, true>(op, a, nfields, st);
+        if constexpr (W > 0) {
+            if (op.MM == 20) return launch_fast_bc<W, H, 20, true>(op, a, nfields, st);
+            if (op.MM == 28) return launch_fast_bc<W, H, 28, true>(op, a, nfields, st);
+        }
         return hipErrorInvalidValue;
     }
     switch (op.MM) {

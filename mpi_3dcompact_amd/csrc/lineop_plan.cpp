@@ -435,16 +435,18 @@ int build_plan(const PlanRequest &rq, Plan &plan, std::string &err) {
     if (per && W > 0 && P < 2) P = 2;
     int M = (n + P - 1) / P;
     int last = n - (P - 1) * M;
-    if (last < std::max(2 * W, 1) || M > mm) { err = "cannot partition line"; return -1; }
     // a line that mm-row chunks do not split evenly: mm-row chunks and one
     // short chunk of the remaining rows, placed second (neither end chunk, which
     // hold the special rows and the ends' halo), when there are at least three
     // chunks and the short one holds both its interface blocks.  Else P chunks
-    // of M rows and a shorter last one (the LDS-tiled kernel only).
+    // of M rows and a shorter last one (the LDS-tiled kernel only; that kernel
+    // takes 16- and 32-row tables, so those requests keep its limits).
     const int rem = n - (P - 1) * mm;
+    const bool short2 = n % mm != 0 && P >= 3 && rem >= std::max(2 * W, 1);
+    if (!(short2 && mm % 16 != 0) && (last < std::max(2 * W, 1) || M > mm)) { err = "cannot partition line"; return -1; }
     plan.cshort = -1;
     plan.lshort = 0;
-    if (n % mm != 0 && P >= 3 && rem >= std::max(2 * W, 1)) {
+    if (short2) {
         plan.cshort = 1;
         plan.lshort = rem;
     }

@@ -1,0 +1,67 @@
+"""Ragged lines in 20- and 28-row chunks: lengths whose remainder over 16 or 32
+rows is too short for the interface blocks (65, 129, 193, ... points), and
+y/z-lines of 257 to 320 points."""
+import numpy as np
+import pytest
+
+import test_plan_cpu as plan
+from oracle import pyoracle as P
+
+OPS = [(0, P.PADE6, 0.0), (0, P.PENTA10, 0.0), (1, P.COMPACT8, 0.49), (1, P.COMPACT10, 0.49), (1, P.COMMN5PADE, 0.0)]
+
+
+@pytest.mark.parametrize("mm", [20, 28])
+@pytest.mark.parametrize("n", [49, 65, 66, 97, 129, 131, 193, 225, 257, 289, 310])
+def test_plan_replay(monkeypatch, n, mm):
+    """The fast kernels' arithmetic over these chunks, replayed on the CPU
+    against the oracle for every banded operator and boundary (bound: the
+    operators' 1e-12)."""
+    def ragged(t):
+        return (t["N"] != t["P"] * t["MM"] and t["P"] >= 3 and t["clen"][1] < t["MM"]
+                and all(c == t["MM"] for i, c in enumerate(t["clen"]) if i != 1))
+
+    monkeypatch.setattr(plan, "ragged", ragged)
+    chunks = -(-n // mm)
+    for cls, kind, af in OPS:
+        W = 2 if (cls, kind) in ((0, P.PENTA10), (1, P.COMMN5PADE)) else 1
+        if n % mm == 0 or chunks < 3 or n - (chunks - 1) * mm < 2 * W:
+            continue
+        for bc in (P.PERIODIC, P.DIRICHLET):
+            dd = 1.0 / n if bc == P.PERIODIC else 1.0 / (n - 1)
+            t = plan.tables(cls, kind, bc, n, dd, af, mm)
+            assert t["MM"] == mm and plan.fast_eligible(t)
+            plan._check(t, (lambda f: P.deriv_line(kind, bc, f, dd)) if cls == 0
+                        else (lambda f: P.filter_line(kind, bc, f, af)), n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [49, 65, 97, 129, 131, 193, 225, 305, 310])
+@pytest.mark.parametrize("d", [0, 1, 2])
+def test_lines_against_oracle(n, d):
+    """Every banded operator on lines of n points among 24 x 24 others, both
+    boundaries, out of place and (filters) in place, at the operators' 1e-12."""
+    import torch
+    from mpi_3dcompact_amd.ops import LineOp
+    dims = [25, 24, 24]
+    dims[d] = n
+    if d:
+        dims[0] = 26  # a last workgroup that is not full
+    dims = tuple(dims)
+    f = np.random.default_rng(n + d).normal(size=dims[::-1])
+    fin = torch.from_numpy(f).cuda()
+    for cls, kind, af in OPS:
+        for bc in (P.PERIODIC, P.DIRICHLET):
+            dd = 1.0 / n if bc == P.PERIODIC else 1.0 / (n - 1)
+            bc3 = [0, 0, 0]
+            bc3[d] = bc
+            op = LineOp.deriv(kind, d, bc, dims, dd) if cls == 0 else LineOp.filter(kind, af, d, bc3, dims)
+            print(f"n={n} dir={d} cls={cls} kind={kind} bc={bc} {op.kernel()}", flush=True)
+            assert not op.kernel().startswith("lineop_kernel<"), op.kernel()
+            want = P.deriv_field(kind, d, bc, f, dd) if cls == 0 else P.filter_field(kind, af, d, bc3, f)
+            out = torch.empty_like(fin)
+            op.apply([fin], [out])
+            if cls == 1:
+                same = fin.clone()
+                op.apply([same], [same])
+                assert torch.equal(same, out)
+            assert np.max(np.abs(out.cpu().numpy() - want)) <= 1e-12 * np.max(np.abs(want)), (cls, kind, bc)
