@@ -46,6 +46,9 @@ hipError_t launch_mlp_reduce(const float *partial, const float *lossp, int nbloc
 struct AdamArgs {
     float lr, b1, b2, eps, c1, c2;
 };
+// launch_mlp_reduce and launch_mlp_adam in one pass (the training loop's)
+hipError_t launch_mlp_reduce_adam(const float *partial, const float *lossp, int nblocks, long n_total, float *loss,
+                                  float *params, float *m, float *v, AdamArgs a, hipStream_t st);
 hipError_t launch_mlp_adam(float *params, float *m, float *v, const float *grad, AdamArgs a, hipStream_t st);
 // Y[n][2] = network(X[n][7]) on standardised values (the register-resident
 // inference path the solver uses)

@@ -48,295 +48,349 @@ __device__ __forceinline__ float gelu_s(float z) {
     return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * (kGc1 + kGc2 * z2)));
 }
 __device__ __forceinline__ float gelu(float z) { return z * gelu_s(z); }
-// d/dz: s + z 2 s (1 - s) k0 (1 + 3 k1 z^2)
-__device__ __forceinline__ float gelu_grad(float z) {
-    const float s = gelu_s(z);
+// d/dz, s = gelu_s(z): s + z 2 s (1 - s) k0 (1 + 3 k1 z^2)
+__device__ __forceinline__ float gelu_grad(float z, float s) {
     return s + z * (2.0f * s * (1.0f - s)) * (kG0 * (1.0f + 3.0f * kG1 * z * z));
 }
 
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63); }
 
+// FP32 -> BF16 by the hardware conversion (round to nearest even, as f2bf for
+// finite values)
+__device__ __forceinline__ short bf16_bits(float v) { return __builtin_bit_cast(short, (__bf16)v); }
+
+__device__ __forceinline__ int kappa(int b, int g, int e) { return 16 * (2 * b + (e >> 2)) + 4 * g + (e & 3); }
+
 // ---------------------------------------------------------------------------
-// training: one workgroup = 4 waves = 64 samples; wave w owns samples
-// 16w..16w+15 in the data products and output-row tile w in the weight
-// products.  Weights and activations are staged in LDS as BF16.
+// training: one workgroup = 4 waves = 64 samples; wave w carries samples
+// 16w .. 16w+15 forward and backward in registers, then forms row tile w of
+// every weight gradient.
+//
+// Products of the passes are computed transposed as in the inference below:
+// D = W h^T (rows = neurons, columns = the wave's 16 samples), so a layer's
+// output tiles are the next layer's B operand once the contraction index is
+// permuted by kappa, forward (W) and backward (W^T) alike, and z, h and dz
+// never leave the registers that form them.  LDS holds what lanes share: the
+// weights as operands (16 bytes per lane and product, converted once per
+// workgroup), and h^T and dz^T as BF16 rows of 64 samples, from which the
+// weight gradients dW = dz^T h read their operands as 16-byte loads.
+//
+// What bounds it: a batch of 8192 is 128 workgroups, one per CU, so the chain
+// of one wave (staging, 60 products, 192 GELUs and their gradients per
+// sample), not the matrix units.  The earlier form staged every operand
+// element by element through 16-bit LDS reads and recomputed z in the backward
+// pass: 56.0 us per batch of 8192, now 13.4.
 // ---------------------------------------------------------------------------
 constexpr int kT = kMlpTile;
-constexpr int kLd0 = 8;  // padded input width (7 features + a zero column)
+constexpr int kTLd = kT + 8;              // samples per LDS row, padded (16-byte rows, no bank conflicts)
+constexpr int kFwdOps = 4 + 8 + 8 + 2;    // W1 t; W2 t,b; W3 t,b; W4 b
+constexpr int kTrainOps = kFwdOps + 4 + 8 + 8;  // then W4^T t; W3^T t,b; W2^T t,b
 
 struct TrainLds {
-    unsigned short w0[kMlpHid * kLd0];     // W1 padded to [64][8]
-    unsigned short w1[kMlpHid * kMlpHid];  // W2
-    unsigned short w2[kMlpHid * kMlpHid];  // W3
-    unsigned short w3[kMlpOut * kMlpHid];  // W4
-    unsigned short a0[kT * kLd0];          // standardised inputs
-    unsigned short act[3][kT * kMlpHid];   // GELU outputs of the hidden layers
-    unsigned short dz[kT * kMlpHid];       // BF16 delta of the current layer's pre-activation
-    unsigned short dyb[kT * kMlpOut];      // BF16 dL/dy
-    float dyf[kT * kMlpOut];               // FP32 dL/dy, then targets before that
-    float red[4 * kMlpHid];                // cross-wave partial sums
-    unsigned char valid[kT];
+    s16x8 w[kTrainOps][64];                  // operands, entry [op][lane]
+    unsigned short a0[16 * kTLd];            // inputs^T (7 features, zero rows above)
+    unsigned short act[3][kMlpHid * kTLd];   // GELU outputs^T
+    unsigned short dz[3][kMlpHid * kTLd];    // deltas^T of the pre-activations
+    unsigned short dy[kMlpOut * kTLd];       // dL/dy^T
+    float b[3][kMlpHid];
+    float red[4][3 * kMlpHid + kMlpOut + 1]; // per-wave sums: three bias gradients, db4, squares
 };
 
-// pre-activation tile (no bias) of hidden/output layer `layer` for samples
-// 16 si.. and neurons 16 nj..: in[s][k] (ld ldin, width kin) times W[j][k]
-__device__ __forceinline__ f32x4 fwd_tile(const unsigned short *in, int ldin, int kin, const unsigned short *W,
-                                          int ldw, int nrows, int si, int nj) {
-    const int l = lane_id(), i = l & 15, g = l >> 4;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < kin; k0 += 32) {
-        s16x8 a, b;
-        const int row_w = 16 * nj + i;
+// the operands of wave w (row and column tile w of every matrix) for the lane
+// (i = lane % 16, g = lane / 16), converted from the FP32 parameters; the
+// four waves' shares are equal and straight-line, so every load is in flight
+// before the first conversion
+__device__ __forceinline__ void stage_train(const float *__restrict__ P, TrainLds &s, int w, int l) {
+    const int i = l & 15, g = l >> 4;
+    float r1[8], c4[2], c3[2][8], c2[2][8];
+    f32x4 r[3][2][2];
+#pragma unroll
+    for (int e = 0; e < kMlpIn; ++e) r1[e] = P[kMlpOffW1 + (16 * w + i) * kMlpIn + e];
+    r1[7] = 0.0f;
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int hi = 0; hi < 2; ++hi) {
+            const int col = 32 * b + 16 * hi + 4 * g;
+            r[0][b][hi] = *reinterpret_cast<const f32x4 *>(P + kMlpOffW2 + (16 * w + i) * kMlpHid + col);
+            r[1][b][hi] = *reinterpret_cast<const f32x4 *>(P + kMlpOffW3 + (16 * w + i) * kMlpHid + col);
+            r[2][b][hi] = *reinterpret_cast<const f32x4 *>(P + kMlpOffW4 + (i < kMlpOut ? i : 0) * kMlpHid + col);
+        }
+#pragma unroll
+    for (int o = 0; o < kMlpOut; ++o) c4[o] = P[kMlpOffW4 + o * kMlpHid + 16 * w + i];
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const int k = k0 + 8 * g + e;
-            a[e] = k < kin ? (short)in[(16 * si + i) * ldin + k] : (short)0;
-            b[e] = (k < kin && row_w < nrows) ? (short)W[row_w * ldw + k] : (short)0;
+            c3[b][e] = P[kMlpOffW3 + kappa(b, g, e) * kMlpHid + 16 * w + i];
+            c2[b][e] = P[kMlpOffW2 + kappa(b, g, e) * kMlpHid + 16 * w + i];
         }
-        acc = mfma(a, b, acc);
-    }
-    return acc;
-}
-
-__device__ __forceinline__ const unsigned short *layer_w(const TrainLds &s, int l) {
-    return l == 0 ? s.w0 : l == 1 ? s.w1 : l == 2 ? s.w2 : s.w3;
-}
-__device__ __forceinline__ const unsigned short *layer_in(const TrainLds &s, int l) {
-    return l == 0 ? s.a0 : s.act[l - 1];
-}
-
-constexpr int kWOff[4] = {kMlpOffW1, kMlpOffW2, kMlpOffW3, kMlpOffW4};
-constexpr int kBOff[4] = {kMlpOffB1, kMlpOffB2, kMlpOffB3, kMlpOffB4};
-
-// column sums over the 64 samples of per-lane values v[t][r] (sample 16w+4g+r,
-// column 16t + l%16) into out[col] (FP32, fixed order); all threads call it
-__device__ void column_sums(TrainLds &s, const float v[4][4], int ncols, float *out) {
-    const int l = lane_id(), w = threadIdx.x >> 6;
+    s16x8 o1, o4;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        float x = ((v[t][0] + v[t][1]) + v[t][2]) + v[t][3];
-        x = x + __shfl_xor(x, 16);
-        x = x + __shfl_xor(x, 32);
-        if (l < 16 && 16 * t + l < ncols) s.red[w * kMlpHid + 16 * t + l] = x;
+    for (int e = 0; e < 8; ++e) {
+        o1[e] = g == 0 ? bf16_bits(r1[e]) : (short)0;
+        o4[e] = g == 0 && e < kMlpOut ? bf16_bits(c4[e < kMlpOut ? e : 0]) : (short)0;
     }
-    __syncthreads();
-    if ((int)threadIdx.x < ncols) {
-        const int c = threadIdx.x;
-        out[c] = ((s.red[c] + s.red[kMlpHid + c]) + s.red[2 * kMlpHid + c]) + s.red[3 * kMlpHid + c];
+    s.w[w][l] = o1;
+    s.w[22 + w][l] = o4;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        s16x8 o2, o3, o2t, o3t, o4r;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            o2[e] = bf16_bits(r[0][b][e >> 2][e & 3]);
+            o3[e] = bf16_bits(r[1][b][e >> 2][e & 3]);
+            o4r[e] = i < kMlpOut ? bf16_bits(r[2][b][e >> 2][e & 3]) : (short)0;
+            o3t[e] = bf16_bits(c3[b][e]);
+            o2t[e] = bf16_bits(c2[b][e]);
+        }
+        s.w[4 + 2 * w + b][l] = o2;
+        s.w[12 + 2 * w + b][l] = o3;
+        if (w == 0) s.w[20 + b][l] = o4r;
+        s.w[26 + 2 * w + b][l] = o3t;
+        s.w[34 + 2 * w + b][l] = o2t;
     }
-    __syncthreads();
+}
+
+// one step of sample_sums: the lane keeps the half of its 2 H values that its
+// bit H selects and adds its partner's
+template <int H>
+__device__ __forceinline__ void fold_samples(float *v, int i) {
+    const bool up = i & H;
+#pragma unroll
+    for (int k = 0; k < H; ++k) {
+        const float keep = up ? v[k + H] : v[k], send = up ? v[k] : v[k + H];
+        v[k] = keep + __shfl_xor(send, H);
+    }
+}
+
+// sums over the 16 samples of the wave of the 16 values v[4t + r] (neuron
+// 16t + 4g + r): a transposing butterfly, after which lane (g, i) holds the
+// sum of value i, neuron 16 (i/4) + 4g + i%4 (fixed order); overwrites v
+__device__ __forceinline__ float sample_sums(float *v, int i) {
+    fold_samples<8>(v, i);
+    fold_samples<4>(v, i);
+    fold_samples<2>(v, i);
+    fold_samples<1>(v, i);
+    return v[0];
+}
+
+// h = GELU(z) as the next layer's operand (BF16) and as rows of the transposed
+// LDS copy; z becomes GELU'(z), which shares the exponential and the reciprocal
+__device__ __forceinline__ void train_activate(f32x4 z[4], s16x8 h[2], unsigned short *rows, int g, int smp) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float zz = z[t][r], sg = gelu_s(zz);
+            const short v = bf16_bits(zz * sg);
+            z[t][r] = gelu_grad(zz, sg);
+            h[t >> 1][4 * (t & 1) + r] = v;
+            rows[(16 * t + 4 * g + r) * kTLd + smp] = (unsigned short)v;
+        }
+}
+
+// dz = dh GELU'(z): FP32 sums over the wave's samples into red, BF16 operand and LDS rows
+__device__ __forceinline__ void train_delta(const f32x4 dh[4], const f32x4 gz[4], s16x8 d[2], unsigned short *rows,
+                                            float *red, int i, int g, int smp) {
+    float v[16];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            v[4 * t + r] = dh[t][r] * gz[t][r];
+            const short q = bf16_bits(v[4 * t + r]);
+            d[t >> 1][4 * (t & 1) + r] = q;
+            rows[(16 * t + 4 * g + r) * kTLd + smp] = (unsigned short)q;
+        }
+    red[16 * (i >> 2) + 4 * g + (i & 3)] = sample_sums(v, i);
+}
+
+// 16 rows of D = A B over the 64 samples, A rows of dz^T, B rows of h^T
+__device__ __forceinline__ f32x4 sample_product(const unsigned short *arow, const unsigned short *brow, int g) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k0 = 0; k0 < kT; k0 += 32)
+        acc = mfma(*reinterpret_cast<const s16x8 *>(arow + k0 + 8 * g), *reinterpret_cast<const s16x8 *>(brow + k0 + 8 * g),
+                   acc);
+    return acc;
 }
 
 __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ P, const float *__restrict__ X,
                                                   const float *__restrict__ Tg, const int *__restrict__ idx,
                                                   long n, float scale, float *__restrict__ partial,
                                                   float *__restrict__ lossp) {
-    __shared__ TrainLds s;
-    const int tid = threadIdx.x, l = lane_id(), w = tid >> 6, g = l >> 4;
+    __shared__ __attribute__((aligned(16))) TrainLds s;
+    const int tid = threadIdx.x, l = lane_id(), w = __builtin_amdgcn_readfirstlane(tid >> 6), i = l & 15, g = l >> 4;
     float *gout = partial + (size_t)blockIdx.x * kMlpParams;
 
-    // ---- stage weights and the sample tile ----
-    for (int q = tid; q < kMlpHid * kLd0; q += 256) {
-        const int j = q / kLd0, k = q % kLd0;
-        s.w0[q] = k < kMlpIn ? f2bf(P[kMlpOffW1 + j * kMlpIn + k]) : (unsigned short)0;
-    }
-    for (int q = tid; q < kMlpHid * kMlpHid; q += 256) {
-        s.w1[q] = f2bf(P[kMlpOffW2 + q]);
-        s.w2[q] = f2bf(P[kMlpOffW3 + q]);
-    }
-    for (int q = tid; q < kMlpOut * kMlpHid; q += 256) s.w3[q] = f2bf(P[kMlpOffW4 + q]);
-    if (tid < kT) {
-        const long q = (long)blockIdx.x * kT + tid;
-        const bool ok = q < n;
-        const long src = ok ? (idx ? (long)idx[q] : q) : 0;
-        s.valid[tid] = ok;
-        for (int k = 0; k < kLd0; ++k)
-            s.a0[tid * kLd0 + k] = (ok && k < kMlpIn) ? f2bf(X[src * kMlpIn + k]) : (unsigned short)0;
-        for (int o = 0; o < kMlpOut; ++o) s.dyf[tid * kMlpOut + o] = ok ? Tg[src * kMlpOut + o] : 0.0f;
+    // ---- this lane's sample (lanes of equal i share it), the operands, the biases ----
+    const int smp = 16 * w + i;
+    const long q = (long)blockIdx.x * kT + smp;
+    const bool ok = q < n;
+    const long src = ok ? (idx ? (long)idx[q] : q) : 0;
+    s16x8 x;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        x[e] = (g == 0 && ok && e < kMlpIn) ? bf16_bits(X[src * kMlpIn + (e < kMlpIn ? e : 0)]) : (short)0;
+    const float t0 = ok ? Tg[src * kMlpOut] : 0.0f, t1 = ok ? Tg[src * kMlpOut + 1] : 0.0f;
+    stage_train(P, s, w, l);
+    if (tid < 3 * kMlpHid)
+        s.b[tid / kMlpHid][tid % kMlpHid] =
+            P[(tid < kMlpHid ? kMlpOffB1 : tid < 2 * kMlpHid ? kMlpOffB2 : kMlpOffB3) + tid % kMlpHid];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {  // rows 4g .. 4g+3 of the transposed inputs: features of lanes g = 0, zeros above
+        const short hi = (short)__shfl((int)x[4 + e], i), lo = (short)__shfl((int)x[e], i);
+        s.a0[(4 * g + e) * kTLd + smp] = (unsigned short)(g == 0 ? lo : g == 1 ? hi : (short)0);
     }
     __syncthreads();
 
-    // ---- forward: hidden layers (wave w: samples 16w.., all 64 neurons) ----
+    // ---- forward ----
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 z[3][4];
+    s16x8 h[2];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) z[0][t] = mfma(s.w[t][l], x, zero);
+#pragma unroll
     for (int layer = 0; layer < 3; ++layer) {
-        const int ldin = layer == 0 ? kLd0 : kMlpHid;
-        const unsigned short *in = layer_in(s, layer), *W = layer_w(s, layer);
+        if (layer > 0) {
 #pragma unroll
-        for (int nj = 0; nj < 4; ++nj) {
-            const f32x4 acc = fwd_tile(in, ldin, ldin, W, ldin, kMlpHid, w, nj);
-            const float b = P[kBOff[layer] + 16 * nj + (l & 15)];
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                s.act[layer][(16 * w + 4 * g + r) * kMlpHid + 16 * nj + (l & 15)] = f2bf(gelu(acc[r] + b));
+            for (int t = 0; t < 4; ++t)
+                z[layer][t] = mfma(s.w[8 * layer - 4 + 2 * t + 1][l], h[1], mfma(s.w[8 * layer - 4 + 2 * t][l], h[0], zero));
         }
-        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) z[layer][t][r] = z[layer][t][r] + s.b[layer][16 * t + 4 * g + r];
+        train_activate(z[layer], h, s.act[layer], g, smp);
     }
-    // ---- output layer, loss, dL/dy ----
-    float sq = 0.0f;
+    // ---- output layer, loss, dL/dy (lanes g = 0 hold the two outputs of their sample) ----
+    const f32x4 y = mfma(s.w[21][l], h[1], mfma(s.w[20][l], h[0], zero));
+    const bool real = g == 0 && ok;
+    const float d0 = real ? (y[0] + P[kMlpOffB4]) - t0 : 0.0f, d1 = real ? (y[1] + P[kMlpOffB4 + 1]) - t1 : 0.0f;
+    const float e0 = scale * d0, e1 = scale * d1;
+    s16x8 d[2];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) d[0][e] = e == 0 ? bf16_bits(e0) : e == 1 ? bf16_bits(e1) : (short)0;
+    if (g == 0) {
+        s.dy[smp] = (unsigned short)d[0][0];
+        s.dy[kTLd + smp] = (unsigned short)d[0][1];
+    }
     {
-        const f32x4 acc = fwd_tile(s.act[2], kMlpHid, kMlpHid, s.w3, kMlpHid, kMlpOut, w, 0);
-        const int o = l & 15;
-        if (o < kMlpOut) {
-            const float b = P[kMlpOffB4 + o];
+        float sq = d0 * d0 + d1 * d1, s0 = e0, s1 = e1;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int smp = 16 * w + 4 * g + r;
-                const float y = acc[r] + b;
-                const float d = s.valid[smp] ? y - s.dyf[smp * kMlpOut + o] : 0.0f;
-                sq = sq + d * d;
-                const float dy = scale * d;
-                s.dyb[smp * kMlpOut + o] = f2bf(dy);
-                s.red[w * kMlpHid + (4 * g + r) * kMlpOut + o] = dy;  // staged, copied below
-            }
+        for (int off = 8; off > 0; off >>= 1) {
+            sq = sq + __shfl_xor(sq, off);
+            s0 = s0 + __shfl_xor(s0, off);
+            s1 = s1 + __shfl_xor(s1, off);
+        }
+        if (l == 0) {
+            s.red[w][3 * kMlpHid] = s0;
+            s.red[w][3 * kMlpHid + 1] = s1;
+            s.red[w][3 * kMlpHid + 2] = sq;
         }
     }
-    // wave sums of squares -> lossp
-    for (int off = 32; off > 0; off >>= 1) sq = sq + __shfl_xor(sq, off);
-    __syncthreads();
-    if (tid < kT * kMlpOut) s.dyf[tid] = s.red[(tid / 32) * kMlpHid + tid % 32];
-    __shared__ float wsq[4];
-    if (l == 0) wsq[w] = sq;
-    __syncthreads();
-    if (tid == 0) lossp[blockIdx.x] = ((wsq[0] + wsq[1]) + wsq[2]) + wsq[3];
-    if (tid < kMlpOut) {  // db4
-        float acc = 0.0f;
-        for (int smp = 0; smp < kT; ++smp) acc = acc + s.dyf[smp * kMlpOut + tid];
-        gout[kMlpOffB4 + tid] = acc;
+    // ---- backward ----
+    f32x4 dh[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) dh[t] = mfma(s.w[22 + t][l], d[0], zero);
+#pragma unroll
+    for (int layer = 2; layer >= 0; --layer) {
+        train_delta(dh, z[layer], d, s.dz[layer], s.red[w] + layer * kMlpHid, i, g, smp);
+        if (layer == 0) break;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int op = (layer == 2 ? 26 : 34) + 2 * t;
+            dh[t] = mfma(s.w[op + 1][l], d[1], mfma(s.w[op][l], d[0], zero));
+        }
     }
+    __syncthreads();
 
-    // ---- backward through the output layer ----
-    {
-        // dW4[o][k] = sum_s dy[s][o] a3[s][k]: wave w -> k tile w
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (int k0 = 0; k0 < kT; k0 += 32) {
-            s16x8 a, b;
+    // ---- gradients: wave w forms rows 16w .. 16w+15 (columns of W4) ----
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int smp = k0 + 8 * g + e;
-                a[e] = (l & 15) < kMlpOut ? (short)s.dyb[smp * kMlpOut + (l & 15)] : (short)0;
-                b[e] = (short)s.act[2][smp * kMlpHid + 16 * w + (l & 15)];
-            }
-            acc = mfma(a, b, acc);
+    for (int layer = 1; layer < 3; ++layer) {
+        const unsigned short *a = s.dz[layer] + (16 * w + i) * kTLd, *in = s.act[layer - 1];
+        float *o = gout + (layer == 1 ? kMlpOffW2 : kMlpOffW3) + (16 * w + 4 * g) * kMlpHid + i;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+            const f32x4 acc = sample_product(a, in + (16 * kt + i) * kTLd, g);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[r * kMlpHid + 16 * kt] = acc[r];
         }
+    }
+    {
+        const f32x4 acc = sample_product(s.dz[0] + (16 * w + i) * kTLd, s.a0 + i * kTLd, g);
+        if (i < kMlpIn) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) gout[kMlpOffW1 + (16 * w + 4 * g + r) * kMlpIn + i] = acc[r];
+        }
+        // rows 2.. of this product repeat row 1 and are not stored
+        const f32x4 acc4 = sample_product(s.dy + (i < kMlpOut ? i : kMlpOut - 1) * kTLd, s.act[2] + (16 * w + i) * kTLd, g);
         if (g == 0) {
 #pragma unroll
-            for (int r = 0; r < kMlpOut; ++r) gout[kMlpOffW4 + r * kMlpHid + 16 * w + (l & 15)] = acc[r];
+            for (int r = 0; r < kMlpOut; ++r) gout[kMlpOffW4 + r * kMlpHid + 16 * w + i] = acc4[r];
         }
     }
-    float dzv[4][4];
-    {
-        // dh3[s][k] = sum_o dy[s][o] W4[o][k], then dz = dh3 * gelu'(z3)
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
-            s16x8 a, b;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int o = 8 * g + e;
-                a[e] = o < kMlpOut ? (short)s.dyb[(16 * w + (l & 15)) * kMlpOut + o] : (short)0;
-                b[e] = o < kMlpOut ? (short)s.w3[o * kMlpHid + 16 * kt + (l & 15)] : (short)0;
-            }
-            const f32x4 dh = mfma(a, b, f32x4{0.f, 0.f, 0.f, 0.f});
-            const f32x4 z = fwd_tile(s.act[1], kMlpHid, kMlpHid, s.w2, kMlpHid, kMlpHid, w, kt);
-            const float bias = P[kMlpOffB3 + 16 * kt + (l & 15)];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) dzv[kt][r] = dh[r] * gelu_grad(z[r] + bias);
-        }
+    if (tid < 3 * kMlpHid + kMlpOut + 1) {
+        const float v = ((s.red[0][tid] + s.red[1][tid]) + s.red[2][tid]) + s.red[3][tid];
+        const int layer = tid / kMlpHid;
+        if (layer < 3) gout[(layer == 0 ? kMlpOffB1 : layer == 1 ? kMlpOffB2 : kMlpOffB3) + tid % kMlpHid] = v;
+        else if (tid < 3 * kMlpHid + kMlpOut) gout[kMlpOffB4 + tid - 3 * kMlpHid] = v;
+        else lossp[blockIdx.x] = v;
     }
-    // dz of layer 2 (W3): store, bias gradient
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s.dz[(16 * w + 4 * g + r) * kMlpHid + 16 * kt + (l & 15)] = f2bf(dzv[kt][r]);
-    column_sums(s, dzv, kMlpHid, gout + kBOff[2]);
+}
 
-    // ---- hidden layers, top down ----
-    for (int layer = 2; layer >= 0; --layer) {
-        const unsigned short *in = layer_in(s, layer);
-        const int kin = layer == 0 ? kMlpIn : kMlpHid;
-        const int ldin = layer == 0 ? kLd0 : kMlpHid;
-        // dW[j][k] = sum_s dz[s][j] in[s][k]: wave w -> row tile w
-        for (int kt = 0; kt < (layer == 0 ? 1 : 4); ++kt) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            for (int k0 = 0; k0 < kT; k0 += 32) {
-                s16x8 a, b;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int smp = k0 + 8 * g + e;
-                    a[e] = (short)s.dz[smp * kMlpHid + 16 * w + (l & 15)];
-                    const int k = 16 * kt + (l & 15);
-                    b[e] = k < ldin ? (short)in[smp * ldin + k] : (short)0;
-                }
-                acc = mfma(a, b, acc);
-            }
-            const int k = 16 * kt + (l & 15);
-            if (k < kin) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) gout[kWOff[layer] + (16 * w + 4 * g + r) * kin + k] = acc[r];
-            }
-        }
-        if (layer == 0) break;
-        // dh[s][k] = sum_j dz[s][j] W[j][k]; dz_prev = dh * gelu'(z_prev)
-        const unsigned short *W = layer_w(s, layer);
-        const unsigned short *inp = layer_in(s, layer - 1), *Wp = layer_w(s, layer - 1);
-        const int ldp = layer - 1 == 0 ? kLd0 : kMlpHid;
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
-            f32x4 dh = {0.f, 0.f, 0.f, 0.f};
-            for (int k0 = 0; k0 < kMlpHid; k0 += 32) {
-                s16x8 a, b;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int j = k0 + 8 * g + e;
-                    a[e] = (short)s.dz[(16 * w + (l & 15)) * kMlpHid + j];
-                    b[e] = (short)W[j * kMlpHid + 16 * kt + (l & 15)];
-                }
-                dh = mfma(a, b, dh);
-            }
-            const f32x4 z = fwd_tile(inp, ldp, ldp, Wp, ldp, kMlpHid, w, kt);
-            const float bias = P[kBOff[layer - 1] + 16 * kt + (l & 15)];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) dzv[kt][r] = dh[r] * gelu_grad(z[r] + bias);
-        }
-        __syncthreads();  // every read of the old dz is done
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                s.dz[(16 * w + 4 * g + r) * kMlpHid + 16 * kt + (l & 15)] = f2bf(dzv[kt][r]);
-        column_sums(s, dzv, kMlpHid, gout + kBOff[layer - 1]);
-    }
+__device__ __forceinline__ void adam_update(float *__restrict__ P, float *__restrict__ m, float *__restrict__ v,
+                                            int p, float gr, const AdamArgs &a) {
+    const float mn = a.b1 * m[p] + (1.0f - a.b1) * gr;
+    const float vn = a.b2 * v[p] + (1.0f - a.b2) * (gr * gr);
+    m[p] = mn;
+    v[p] = vn;
+    const float mh = mn / a.c1, vh = vn / a.c2;
+    P[p] = P[p] - a.lr * mh / (sqrtf(vh) + a.eps);
 }
 
 // Sum of the nb partial gradients of every parameter and of the partial
 // losses, in a fixed order (the result does not depend on scheduling): a
-// workgroup takes 64 parameters, its four waves each sum a quarter of the
-// partials in order (rows of 64 consecutive floats), and the four sums are
-// added in wave order.  Workgroup 0 also sums the partial losses: strided
-// per thread, then a fixed tree.  (One thread per parameter summing all nb
-// partials kept 35 workgroups busy and took 35 us per batch.)
-constexpr int kReduceCols = 64;
-__global__ __launch_bounds__(256) void k_mlp_reduce(const float *__restrict__ partial,
+// workgroup takes 64 parameters, its eight waves each sum an eighth of the
+// partials in order (rows of 64 consecutive floats, 16 loads in flight), and
+// the eight sums are added in wave order.  Workgroup 0 also sums the partial
+// losses: strided per thread, then a fixed tree.  With ADAM the thread that
+// holds a parameter's gradient updates it in the same pass (grad null: not
+// written), which saves the training loop a launch per batch.
+constexpr int kReduceCols = 64, kReduceWaves = 8;
+template <bool ADAM>
+__global__ __launch_bounds__(512) void k_mlp_reduce(const float *__restrict__ partial,
                                                     const float *__restrict__ lossp, int nb, float inv_norm,
-                                                    float *__restrict__ grad, float *__restrict__ loss) {
-    __shared__ float part[4][kReduceCols];
-    __shared__ float lsum[256];
+                                                    float *__restrict__ grad, float *__restrict__ loss,
+                                                    float *__restrict__ P, float *__restrict__ m,
+                                                    float *__restrict__ v, AdamArgs a) {
+    __shared__ float part[kReduceWaves][kReduceCols];
+    __shared__ float lsum[512];
     const int t = threadIdx.x % kReduceCols, g = threadIdx.x / kReduceCols;
     const int p = blockIdx.x * kReduceCols + t;
-    const int per = (nb + 3) / 4, b0 = g * per, b1 = b0 + per < nb ? b0 + per : nb;
+    const int per = (nb + kReduceWaves - 1) / kReduceWaves, b0 = g * per, b1 = b0 + per < nb ? b0 + per : nb;
     float acc = 0.0f;
     if (p < kMlpParams) {
-#pragma unroll 8
+#pragma unroll 16
         for (int b = b0; b < b1; ++b) acc = acc + partial[(size_t)b * kMlpParams + p];
     }
     part[g][t] = acc;
     if (blockIdx.x == 0) {
         float l = 0.0f;
-        for (int b = threadIdx.x; b < nb; b += 256) l = l + lossp[b];
+        for (int b = threadIdx.x; b < nb; b += 512) l = l + lossp[b];
         lsum[threadIdx.x] = l;
     }
     __syncthreads();
-    if (g == 0 && p < kMlpParams) grad[p] = ((part[0][t] + part[1][t]) + part[2][t]) + part[3][t];
+    if (g == 0 && p < kMlpParams) {
+        float gr = part[0][t];
+#pragma unroll
+        for (int k = 1; k < kReduceWaves; ++k) gr = gr + part[k][t];
+        if (grad) grad[p] = gr;
+        if (ADAM) adam_update(P, m, v, p, gr, a);
+    }
     if (blockIdx.x == 0) {
-        for (int h = 128; h > 0; h >>= 1) {
+        for (int h = 256; h > 0; h >>= 1) {
             if (threadIdx.x < h) lsum[threadIdx.x] = lsum[threadIdx.x] + lsum[threadIdx.x + h];
             __syncthreads();
         }
@@ -347,14 +401,7 @@ __global__ __launch_bounds__(256) void k_mlp_reduce(const float *__restrict__ pa
 __global__ void k_mlp_adam(float *__restrict__ P, float *__restrict__ m, float *__restrict__ v,
                            const float *__restrict__ grad, AdamArgs a) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= kMlpParams) return;
-    const float gr = grad[p];
-    const float mn = a.b1 * m[p] + (1.0f - a.b1) * gr;
-    const float vn = a.b2 * v[p] + (1.0f - a.b2) * (gr * gr);
-    m[p] = mn;
-    v[p] = vn;
-    const float mh = mn / a.c1, vh = vn / a.c2;
-    P[p] = P[p] - a.lr * mh / (sqrtf(vh) + a.eps);
+    if (p < kMlpParams) adam_update(P, m, v, p, grad[p], a);
 }
 
 // ---------------------------------------------------------------------------
@@ -372,8 +419,6 @@ struct InferW {
     float b1[16], b2[16], b3[16];  // [t * 4 + r]: neuron 16t + 4g + r
     float b4[4];                   // [r]: output 4g + r
 };
-
-__device__ __forceinline__ int kappa(int b, int g, int e) { return 16 * (2 * b + (e >> 2)) + 4 * g + (e & 3); }
 
 __device__ void load_infer(const float *__restrict__ P, InferW &W) {
     const int l = lane_id(), i = l & 15, g = l >> 4;
@@ -604,10 +649,6 @@ __device__ void stage_infer(const float *__restrict__ P, InferLds &s) {
     if (threadIdx.x < 4) s.b4[threadIdx.x] = threadIdx.x < kMlpOut ? P[kMlpOffB4 + threadIdx.x] : 0.0f;
     __syncthreads();
 }
-
-// FP32 -> BF16 by the hardware conversion (round to nearest even, as f2bf for
-// finite values)
-__device__ __forceinline__ short bf16_bits(float v) { return __builtin_bit_cast(short, (__bf16)v); }
 
 __device__ __forceinline__ void activate_lds(const f32x4 acc[4], const float *bias, int g, s16x8 h[2]) {
 #pragma unroll
@@ -865,8 +906,16 @@ hipError_t launch_mlp_grad_partials(const float *params, const float *X, const f
 hipError_t launch_mlp_reduce(const float *partial, const float *lossp, int nblocks, long n_total, float *grad,
                              float *loss, hipStream_t st) {
     const float inv_norm = (float)(1.0 / ((double)n_total * kMlpOut));
-    hipLaunchKernelGGL(k_mlp_reduce, dim3((kMlpParams + kReduceCols - 1) / kReduceCols), dim3(256), 0, st, partial,
-                       lossp, nblocks, inv_norm, grad, loss);
+    hipLaunchKernelGGL(k_mlp_reduce<false>, dim3((kMlpParams + kReduceCols - 1) / kReduceCols), dim3(512), 0, st,
+                       partial, lossp, nblocks, inv_norm, grad, loss, nullptr, nullptr, nullptr, AdamArgs{});
+    return hipGetLastError();
+}
+
+hipError_t launch_mlp_reduce_adam(const float *partial, const float *lossp, int nblocks, long n_total, float *loss,
+                                  float *params, float *m, float *v, AdamArgs a, hipStream_t st) {
+    const float inv_norm = (float)(1.0 / ((double)n_total * kMlpOut));
+    hipLaunchKernelGGL(k_mlp_reduce<true>, dim3((kMlpParams + kReduceCols - 1) / kReduceCols), dim3(512), 0, st,
+                       partial, lossp, nblocks, inv_norm, nullptr, loss, params, m, v, a);
     return hipGetLastError();
 }
 

@@ -27,7 +27,6 @@ Closure::Closure(uint64_t seed) {
     params = dev_alloc<float>(kMlpParams, "closure parameters");
     m_ = dev_alloc<float>(kMlpParams, "closure moments");
     v_ = dev_alloc<float>(kMlpParams, "closure moments");
-    grad_ = dev_alloc<float>(kMlpParams, "closure gradient");
     std::vector<float> h(kMlpParams, 0.0f);
     std::mt19937_64 rng(seed);
     const int fan[4] = {kMlpIn, kMlpHid, kMlpHid, kMlpHid};
@@ -47,7 +46,7 @@ Closure::Closure(uint64_t seed) {
 
 Closure::~Closure() {
     (void)hipDeviceSynchronize();
-    for (void *p : {(void *)params, (void *)m_, (void *)v_, (void *)grad_, (void *)loss_, (void *)partial_,
+    for (void *p : {(void *)params, (void *)m_, (void *)v_, (void *)loss_, (void *)partial_,
                     (void *)lossp_, (void *)idx_})
         if (p) (void)hipFree(p);
 }
@@ -102,12 +101,16 @@ double Closure::gradient(const float *X, const float *T, long n, float *grad, hi
 
 // Adam (Kingma & Ba 2015), beta1 0.9, beta2 0.999, eps 1e-8; bias corrections
 // formed in FP64 and rounded to FP32
-void Closure::adam(const float *grad, float lr, hipStream_t st) {
+AdamArgs Closure::next_adam(float lr) {
     ++adam_t;
     AdamArgs a{lr, 0.9f, 0.999f, 1e-8f, 0.0f, 0.0f};
     a.c1 = (float)(1.0 - std::pow((double)a.b1, adam_t));
     a.c2 = (float)(1.0 - std::pow((double)a.b2, adam_t));
-    hip_check(launch_mlp_adam(params, m_, v_, grad, a, st), "closure adam");
+    return a;
+}
+
+void Closure::adam(const float *grad, float lr, hipStream_t st) {
+    hip_check(launch_mlp_adam(params, m_, v_, grad, next_adam(lr), st), "closure adam");
 }
 
 void Closure::train(const float *X, const float *T, long n, int epochs, int batch, float lr, uint64_t seed,
@@ -132,8 +135,8 @@ void Closure::train(const float *X, const float *T, long n, int epochs, int batc
             const int nblk = (int)((nb_s + kMlpTile - 1) / kMlpTile);
             hip_check(launch_mlp_grad_partials(params, X, T, idx_ + b * batch, nb_s, nb_s, partial_, lossp_, st),
                       "closure gradient");
-            hip_check(launch_mlp_reduce(partial_, lossp_, nblk, nb_s, grad_, loss_ + b, st), "closure gradient sum");
-            adam(grad_, lr, st);
+            hip_check(launch_mlp_reduce_adam(partial_, lossp_, nblk, nb_s, loss_ + b, params, m_, v_, next_adam(lr), st),
+                      "closure gradient sum");
         }
         hip_check(hipMemcpyAsync(bl.data(), loss_, sizeof(float) * (size_t)nbatches, hipMemcpyDeviceToHost, st),
                   "closure losses");

@@ -37,6 +37,7 @@ class Closure {
     double gradient(const float *X, const float *T, long n, float *grad, hipStream_t st);
     // one Adam step with a given gradient (device)
     void adam(const float *grad, float lr, hipStream_t st);
+    AdamArgs next_adam(float lr);  // counts the update and forms its bias corrections
     // epochs of shuffled minibatch Adam; losses[e] = mean minibatch loss of epoch e
     void train(const float *X, const float *T, long n, int epochs, int batch, float lr, uint64_t seed,
                double *losses, hipStream_t st);
@@ -45,7 +46,7 @@ class Closure {
     void load(const std::string &path);
 
   private:
-    float *m_ = nullptr, *v_ = nullptr, *grad_ = nullptr, *loss_ = nullptr;
+    float *m_ = nullptr, *v_ = nullptr, *loss_ = nullptr;
     float *partial_ = nullptr, *lossp_ = nullptr;
     int *idx_ = nullptr;
     long idx_cap_ = 0, part_blocks_ = 0, loss_cap_ = 0;
