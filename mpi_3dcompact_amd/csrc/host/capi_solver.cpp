@@ -240,16 +240,18 @@ int mc3d_solver_run(mc3d_solver *s) {
 
 int mc3d_solver_field_device(mc3d_solver *s, const char *name, double **dev_ptr) {
     if (!s || !name || !dev_ptr) return mc3d::fail(MC3D_EINVAL, "null argument");
-    double *p = s->cs->field_by_name(name);
+    double *p = nullptr;
+    if (const int rc = guarded([&] { p = s->cs->expose_field(name); })) return rc;
     if (!p) return mc3d::fail(MC3D_EINVAL, std::string("unknown field ") + name);
     *dev_ptr = p;
     return MC3D_OK;
 }
 
 int mc3d_solver_get_field(mc3d_solver *s, const char *name, double *host_out) {
+    if (!s || !name) return mc3d::fail(MC3D_EINVAL, "null argument");
     double *p = nullptr;
-    int rc = mc3d_solver_field_device(s, name, &p);
-    if (rc) return rc;
+    if (const int rc = guarded([&] { p = s->cs->field_by_name(name); })) return rc;
+    if (!p) return mc3d::fail(MC3D_EINVAL, std::string("unknown field ") + name);
     if (!host_out) return mc3d::fail(MC3D_EINVAL, "null output");
     return guarded([&] {
         mc3d::hip_check(hipMemcpyAsync(host_out, p, sizeof(double) * s->cs->N, hipMemcpyDeviceToHost,

@@ -163,7 +163,7 @@ VremanSGS::VremanSGS(CurvilinearCSolver *c) {
 
 void VremanSGS::getSGSViscosity(const double *const dU[3], const double *const dV[3],
                                 const double *const dW[3], const double *rho) {
-    cs->timed("k_vreman", 21.0, [&] {
+    cs->timed("k_vreman", 11.0 + cs->metric_fields_, [&] {
         hip_check(launch_vreman(dU, dV, dW, cs->msh, rho, mu_sgs, cs->dom.dx, cs->dom.dy, cs->dom.dz,
                                 cs->N, cs->st),
                   "vreman");
@@ -432,6 +432,7 @@ CurvilinearCSolver::CurvilinearCSolver(const Options &o, hipStream_t s, int memb
     hip_check(hipMalloc(&slab_, slab_bytes_), "field allocation");
     for (int k = 0; k < 10; ++k) Jm[k] = alloc_field();
     msh = Metrics{Jm[0], Jm[1], Jm[2], Jm[3], Jm[4], Jm[5], Jm[6], Jm[7], Jm[8], Jm[9]};
+    msh.plane = (unsigned)(dom.gNx * dom.gNy);
     for (int q = 0; q < 5; ++q) { r1.q[q] = alloc_field(); rk_.q[q] = alloc_field(); k2.q[q] = alloc_field(); r2.q[q] = alloc_field(); }
     pr = Prim{alloc_field(), alloc_field(), alloc_field(), alloc_field(), alloc_field(),
               alloc_field(), alloc_field(), alloc_field(), alloc_field(), alloc_field()};
@@ -449,6 +450,10 @@ CurvilinearCSolver::CurvilinearCSolver(const Options &o, hipStream_t s, int memb
     hip_check(hipMalloc(&p, sizeof(StepScalars) * members), "scalar allocation");
     extra_.push_back(p);
     sc = static_cast<StepScalars *>(p);
+    hip_check(hipMalloc(&p, sizeof(int)), "metric flag");
+    extra_.push_back(p);
+    msh.varies = planes_vary_ = static_cast<int *>(p);
+    checkMetricPlanes();
     const std::vector<StepScalars> s0((size_t)members, StepScalars{opt.dt, opt.CFL, opt.time, 0.0});
     hip_check(hipMemcpy(sc, s0.data(), sizeof(StepScalars) * members, hipMemcpyHostToDevice), "scalar init");
     if (members > 1) {
@@ -542,6 +547,7 @@ CurvilinearCSolver::CurvilinearCSolver(const Options &o, hipStream_t s, SgsOnly 
     hip_check(hipMalloc(&slab_, slab_bytes_), "field allocation");
     tmp[9] = alloc_field();
     msh = Metrics{t.J, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+    msh.plane = (unsigned)(dom.gNx * dom.gNy);
     void *p = nullptr;
     hip_check(hipMalloc(&p, sizeof(double) * std::max<size_t>(4096, (size_t)cfl_blocks(dom.gN))),
               "scratch allocation");
@@ -574,9 +580,31 @@ double *CurvilinearCSolver::alloc_field() {
     return reinterpret_cast<double *>(static_cast<char *>(slab_) + off);
 }
 
+// The flag lives on the device and is set again with every change of the
+// metrics, so captured steps read the current one.  A metric field whose device
+// address the caller holds may change at any time: its planes count as different.
+void CurvilinearCSolver::checkMetricPlanes() {
+    hip_check(metrics_exposed_ ? launch_set_int(planes_vary_, 1, st) : launch_metric_planes(msh, planes_vary_, N, st),
+              "metric planes");
+    int varies = 1;  // a copy for the byte counts of the launch timings
+    hip_check(hipMemcpyAsync(&varies, planes_vary_, sizeof(int), hipMemcpyDeviceToHost, st), "metric planes");
+    hip_check(hipStreamSynchronize(st), "metric planes");
+    metric_fields_ = varies ? 10.0 : 0.0;
+}
+
+double *CurvilinearCSolver::expose_field(const std::string &name) {
+    double *p = field_by_name(name);
+    if (std::find(Jm, Jm + 10, p) != Jm + 10 && p) {
+        metrics_exposed_ = true;
+        checkMetricPlanes();
+    }
+    return p;
+}
+
 void CurvilinearCSolver::set_metrics_host(const double *const m[10]) {
     for (int k = 0; k < 10; ++k)
         hip_check(hipMemcpyAsync(Jm[k], m[k], sizeof(double) * N, hipMemcpyHostToDevice, st), "metric upload");
+    checkMetricPlanes();
     hip_check(hipStreamSynchronize(st), "metric upload");
 }
 
@@ -628,6 +656,7 @@ void CurvilinearCSolver::setMemberMetrics(int b, const double *const m[10]) {
     for (int k = 0; k < 10; ++k)
         hip_check(hipMemcpyAsync(Jm[k] + off, m[k], sizeof(double) * dom.gN, hipMemcpyHostToDevice, st),
                   "metric upload");
+    checkMetricPlanes();
     hip_check(hipStreamSynchronize(st), "metric upload");
 }
 
@@ -726,6 +755,7 @@ void CurvilinearCSolver::solveForJacobians(const double *x, const double *y, con
     double *out[10];
     for (int k = 0; k < 10; ++k) out[k] = msh_rw(k);
     solve_for_jacobians(dv, m, x, y, z, out, st);
+    checkMetricPlanes();
 }
 
 void CurvilinearCSolver::set_mesh_host(const double *x, const double *y, const double *z) {
@@ -1058,8 +1088,8 @@ void CurvilinearCSolver::flux() {
     // 1: mu_sgs with k_sgs from Pr_t (Vreman); 2: mu_sgs and k_sgs fields (DSM, learned)
     fa.les = opt.lesModel == Options::NOMODEL ? 0 : opt.lesModel == Options::VREMAN ? 1 : 2;
     fa.Pr_t = Pr_t;
-    // read: 12 derivatives, 10 metrics, U V W p mu, 5 conserved (+ mu_sgs, k_sgs); written: 15
-    const double flux_fields = 32.0 + 15.0 + (fa.les ? 1.0 : 0.0) + (fa.les == 2 ? 1.0 : 0.0);
+    // read: 12 derivatives, metrics, U V W p mu, 5 conserved (+ mu_sgs, k_sgs); written: 15
+    const double flux_fields = 22.0 + metric_fields_ + 15.0 + (fa.les ? 1.0 : 0.0) + (fa.les == 2 ? 1.0 : 0.0);
     timed("k_flux", flux_fields, [&] { hip_check(launch_flux(fa, ig, N, st), "flux"); });
     // divergence: xi of the _1 fluxes, then eta of _2 and zeta of _3 added in
     // (src/CurvilinearCSolver_Core.cpp:763-773 with the sums of :810,839,...)
@@ -1095,11 +1125,13 @@ void CurvilinearCSolver::stage_update(int op, double a, double b, double c) {
     ra.pr = pr;
     ra.g = ig;
     ra.bc = rkBoundaryArgs();
+    ra.last = rkLast ? 1 : 0;
     eos_done_ = ra.eos != 0;
-    // fields: div (5) + J + previous momentum k2 (3) read, k2 (5) written, plus the
-    // registers, plus U V W p T mu sos written when the update rides along
+    // fields: div (5) + J + previous momentum k2 (3) read, k2 (3, all 5 by the
+    // last stage) written, plus the registers, plus U V W p T mu written when the
+    // update rides along
     static const double reg[9] = {10, 15, 15, 15, 20, 10, 15, 20, 20};
-    timed("k_rhs_rk", 14.0 + reg[op] + (ra.eos ? 7.0 : 0.0),
+    timed("k_rhs_rk", 12.0 + (ra.last ? 2.0 : 0.0) + reg[op] + (ra.eos ? 6.0 : 0.0),
           [&] { hip_check(launch_rhs_rk(ra, N, st), "stage update"); });
 }
 

@@ -319,6 +319,9 @@ class CurvilinearCSolver {
     // device fields (one slab)
     Metrics msh{};
     double *Jm[10] = {};
+    int *planes_vary_ = nullptr;     // Metrics::varies
+    double metric_fields_ = 10.0;    // metric fields k_flux and k_vreman stream (0: the first plane)
+    bool metrics_exposed_ = false;   // a metric field's address was handed out
     Cons r1{}, rk_{}, k2{}, r2{};
     Prim pr{};
     double *dU[3] = {}, *dV[3] = {}, *dW[3] = {}, *dT[3] = {};
@@ -337,6 +340,10 @@ class CurvilinearCSolver {
 
     double *alloc_field();
     void set_metrics_host(const double *const m[10]);
+    // field_by_name for callers that keep the address
+    double *expose_field(const std::string &name);
+    // sets *planes_vary_ from the metric fields
+    void checkMetricPlanes();
     // metrics from mesh coordinates (device x, y, z), src/AbstractSingleBlockMesh.cpp:23-1309
     void solveForJacobians(const double *x, const double *y, const double *z);
     void set_mesh_host(const double *x, const double *y, const double *z);

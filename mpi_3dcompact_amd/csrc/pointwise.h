@@ -26,6 +26,12 @@ __device__ __forceinline__ double member_mu_ref(const Gas &g, long ip) {
 
 struct Metrics {
     const double *J, *J11, *J12, *J13, *J21, *J22, *J23, *J31, *J32, *J33;
+    // points of a z-plane, and whether the planes differ (a device flag,
+    // launch_metric_planes; null: they may).  Where *varies is 0 every plane
+    // repeats the first (a mesh extruded along z: a box, a channel stretched
+    // towards its walls, an O-grid), and k_flux and k_vreman read that plane
+    unsigned plane = 0;
+    const int *varies = nullptr;
 };
 
 struct Cons {  // one register set of conserved variables: rho, rhoU, rhoV, rhoW, rhoE
@@ -78,6 +84,10 @@ struct RkArgs {
     int op;
     double a, b, c;        // stage coefficients
     int eos;               // also update the non-conserved data from the new rk state
+    // last stage of a step: k2 of rho and rhoE are written (no stage reads
+    // them; they are the step's results), as the speed of sound is by the
+    // update after it (only the next step's CFL reads it)
+    int last;
     Prim pr;
     Gas g;
     RkBc bc;
@@ -110,6 +120,10 @@ hipError_t launch_cfl_finish(const double *partial, int nblocks, StepScalars *sc
 // the same maxima into out[2 b] = cfl / maxspeed, out[2 b + 1] = maxspeed of each member
 hipError_t launch_cfl_out(const double *partial, int nblocks, int nmember, double cfl, double *out,
                           hipStream_t st);
+// *varies = 1 if any of the ten metric fields (n points) differs in any bit
+// between z-planes of `plane` points, else 0
+hipError_t launch_metric_planes(const Metrics &m, int *varies, long n, hipStream_t st);
+hipError_t launch_set_int(int *p, int v, hipStream_t st);
 hipError_t launch_flux(const FluxArgs &a, Gas g, long n, hipStream_t st);
 hipError_t launch_rhs_rk(const RkArgs &a, long n, hipStream_t st);
 hipError_t launch_vreman(const double *const dU[3], const double *const dV[3],

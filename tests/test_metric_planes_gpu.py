@@ -1,0 +1,78 @@
+"""The pointwise kernels over meshes that repeat their first z-plane: the same
+bits as with every point's own metric terms, and no plane is taken for repeated
+that is not."""
+import numpy as np
+import pytest
+
+from mpi_3dcompact_amd import hit
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+
+
+def run(dims, metrics, own, again=None, steps=2):
+    """Conserved and k2 fields after some steps; own: every point streams its own
+    metric terms (a metric field's address was handed out); again: metrics set
+    after the first step."""
+    from mpi_3dcompact_amd.solver import Solver
+    shape = dims[::-1]
+    s = Solver(hit.options_text(dims[0], fd="PADE6", filt="COMPACT8", rk="KENRK4", les="VREMAN", les_avg="NONE",
+                                mu_ref=1e-3, dims=dims), shape)
+    s.set_metrics(metrics)
+    r = np.random.default_rng(5)
+    s.set_initial(dict(rho=1.0 + 0.1 * r.random(shape), p=1.0 / 1.4 + 0.1 * r.random(shape),
+                       **{k: 0.2 * r.standard_normal(shape) for k in "UVW"}))
+    if own:
+        s.device_ptr("J11")
+    s.step(1)
+    if again is not None:
+        s.set_metrics(again)
+    s.step(steps - 1)
+    return {n: s.field(n) for n in ("rho", "rhoU", "rhoV", "rhoW", "rhoE", "rhok2", "rhoUk2", "rhoEk2", "sos", "mu_sgs")}
+
+
+def extruded(dims):
+    """Non-diagonal metrics that depend on (x, y) alone."""
+    nx, ny, nz = dims
+    r = np.random.default_rng(2)
+    base = hit.identity_metrics(8)
+    return [np.broadcast_to(b[0, 0, 0] * (1.0 + 0.05 * r.random((ny, nx))) + 0.001 * r.random((ny, nx)),
+                            (nz, ny, nx)).copy() for b in base]
+
+
+@pytest.mark.parametrize("dims", [(32, 32, 32), (13, 12, 36), (64, 20, 16)])
+def test_repeated_planes_give_the_same_bits(dims):
+    m = extruded(dims)
+    a, b = run(dims, m, False), run(dims, m, True)
+    for k in a:
+        assert np.all(np.isfinite(a[k])) and np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("field", [0, 2, 9])
+def test_one_point_of_the_last_plane(field):
+    """A single value off by one bit in the last plane makes the planes differ."""
+    dims = (32, 16, 16)
+    m = extruded(dims)
+    m[field][-1, -1, -1] = np.nextafter(m[field][-1, -1, -1], 10.0) * (1.0 + 0.01)
+    a, b = run(dims, m, False), run(dims, m, True)
+    for k in a:
+        assert np.array_equal(a[k], b[k]), k
+    c = run(dims, extruded(dims), False)
+    assert not np.array_equal(a["rhoE"], c["rhoE"])
+
+
+def test_metrics_set_again():
+    """New metrics between steps are looked at again, in both directions."""
+    dims = (32, 16, 16)
+    m, v = extruded(dims), extruded(dims)
+    v[5][3:] *= 1.02
+    for first, second in ((m, v), (v, m)):
+        a, b = run(dims, first, False, again=second), run(dims, first, True, again=second)
+        for k in a:
+            assert np.array_equal(a[k], b[k]), k
