@@ -75,6 +75,29 @@ int rotate(int layout, int dir, const int dims[3], const int bc3[3], int vd[3], 
     return MC3D_OK;
 }
 
+// Rows per chunk of evenly chunked y- and z-lines of banded operators, or 0 for
+// the plan's own choice (32 or 16 rows).  A workgroup is one wave per chunk, so
+// the chunk count sets how well workgroups pack into a CU's wave slots: 6, 8,
+// 12 or 16 chunks of 20, 24 or 28 rows (or four of 24) beat the 5 to 15 chunks
+// of 32 or 16 rows the same line splits into.  Four fields, y, 32 (or 16) rows
+// against these: 144 points Penta10 113 -> 93 us, 160 Compact10 104 -> 82, 192
+// Compact10 99 -> 84 and Penta10 101 -> 85, 224 CommN5Pade 105 -> 91, 240 Penta10
+// 124 -> 93, 288 Penta10 127 -> 96, 320 Pade6 101 -> 93, 384 Penta10 107 -> 104,
+// 448 105 -> 97, 96 91 -> 83.  (28 x 4 at 112 points was mixed; 128 and 256
+// points have no such split and keep 32.)  64 points: four chunks of 16 rows
+// instead of two of 32, which leave a 64^3 box 512 waves for 1024 SIMDs
+// (four fields: Pade6 7.7 -> 6.9 us, Penta10 8.6 -> 7.6, Compact10 10.0 -> 7.6).
+int strided_rows(int cls, int kind, int n) {
+    const bool banded = cls == mc3d::kDeriv ? kind != MC3D_CD2 : kind != MC3D_COMMN5EXP;
+    if (!banded || n % 16 != 0) return 0;
+    if (n / 32 == 2) return n % 32 ? 0 : 16;
+    for (int mm : {24, 28, 20}) {
+        const int P = n / mm;
+        if (n % mm == 0 && (P == 6 || P == 8 || P == 12 || P == 16 || (P == 4 && mm == 24))) return mm;
+    }
+    return 0;
+}
+
 int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[3], double dd,
            double alphaF, int nbatch, const mc3d::LineTune &tune, mc3d_lineop **out) {
     if (!out) return mc3d::fail(MC3D_EINVAL, "null output handle");
@@ -104,10 +127,12 @@ int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
     // CU; 16-row chunks double them, and measured faster for every x operator:
     // the Penta10 derivative of 256-point lines inside the LES step 3.3 ->
     // 2.9 ms), then the plan's own choice (32 rows or an even 8..28-row split),
-    // which also serves lines too long for 16-row chunks in one workgroup.
+    // which also serves lines too long for 16-row chunks in one workgroup;
+    // for y- and z-lines strided_rows first.
     // When none is fast, 16-row chunks for the LDS-tiled kernel.
     int cand[2] = {tune.mm, -1};
     if (!tune.mm && dir == 0 && dims[0] % 16 == 0) cand[0] = 16, cand[1] = 0;
+    if (!tune.mm && dir != 0) cand[0] = strided_rows(cls, kind, dims[dir]), cand[1] = 0;
     auto plan_with = [&](int mm) -> int {
         mc3d::PlanRequest rq{cls, kind, bc, dims[dir], dd, alphaF, mm};
         op->plan = mc3d::Plan();

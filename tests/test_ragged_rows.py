@@ -1,6 +1,6 @@
 """Ragged lines in 20- and 28-row chunks: lengths whose remainder over 16 or 32
 rows is too short for the interface blocks (65, 129, 193, ... points), and
-y/z-lines of 257 to 320 points."""
+y/z-lines of 257 to 320 points; and the chunk rows of evenly chunked y/z-lines."""
 import numpy as np
 import pytest
 
@@ -64,4 +64,31 @@ def test_lines_against_oracle(n, d):
                 same = fin.clone()
                 op.apply([same], [same])
                 assert torch.equal(same, out)
+            assert np.max(np.abs(out.cpu().numpy() - want)) <= 1e-12 * np.max(np.abs(want)), (cls, kind, bc)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,mm", [(64, 16), (96, 24), (144, 24), (160, 20), (224, 28), (240, 20), (336, 28), (448, 28),
+                                  (112, 16), (128, 32), (256, 32)])
+@pytest.mark.parametrize("d", [1, 2])
+def test_even_rows(n, mm, d):
+    """The rows per chunk that evenly chunked y/z-lines take, and every banded
+    operator over them against the oracle at 1e-12."""
+    import torch
+    from mpi_3dcompact_amd.ops import LineOp
+    dims = [70, 12, 12]
+    dims[d] = n
+    dims = tuple(dims)
+    f = np.random.default_rng(n + d).normal(size=dims[::-1])
+    fin = torch.from_numpy(f).cuda()
+    for cls, kind, af in OPS:
+        for bc in (P.PERIODIC, P.DIRICHLET):
+            dd = 1.0 / n if bc == P.PERIODIC else 1.0 / (n - 1)
+            bc3 = [0, 0, 0]
+            bc3[d] = bc
+            op = LineOp.deriv(kind, d, bc, dims, dd) if cls == 0 else LineOp.filter(kind, af, d, bc3, dims)
+            assert f", {mm}, " in op.kernel() and op.kernel().startswith("lineop_strided<"), op.kernel()
+            want = P.deriv_field(kind, d, bc, f, dd) if cls == 0 else P.filter_field(kind, af, d, bc3, f)
+            out = torch.empty_like(fin)
+            op.apply([fin], [out])
             assert np.max(np.abs(out.cpu().numpy() - want)) <= 1e-12 * np.max(np.abs(want)), (cls, kind, bc)
