@@ -98,6 +98,23 @@ int strided_rows(int cls, int kind, int n) {
     return 0;
 }
 
+// Rows per chunk with which lineop_contig_groups takes x-lines of n points of a
+// banded operator (half bandwidth W), Dirichlet or ragged, or 0: four or eight
+// chunks, whose waves spread evenly over a CU's SIMDs (the fewest rows that give
+// at most so many; 144 points: eight chunks of 20 rows 3.6-4.0 TB/s, six of 24
+// 2.9-3.4).  113 to 128 points are eight 16-row chunks, which the whole tile serves
+// as well.  Fewer than 1024 lines leave most of the chip idle either way and keep
+// the whole tile, as do shorter lines, of which several tiles fit a CU.
+int grouped_rows(int n, int W, long nlines) {
+    if (n < 96 || n > 256 || nlines < 1024 || (n > 112 && n <= 128)) return 0;
+    const int chunks = n <= 112 ? 4 : 8;
+    for (int mm : {20, 24, 28, 32}) {
+        const int P = (n + mm - 1) / mm, rem = n - (P - 1) * mm;
+        if (P <= chunks && P >= 3 && rem >= 2 * W) return mm;
+    }
+    return 0;
+}
+
 int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[3], double dd,
            double alphaF, int nbatch, const mc3d::LineTune &tune, mc3d_lineop **out) {
     if (!out) return mc3d::fail(MC3D_EINVAL, "null output handle");
@@ -133,6 +150,7 @@ int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
     int cand[2] = {tune.mm, -1};
     if (!tune.mm && dir == 0 && dims[0] % 16 == 0) cand[0] = 16, cand[1] = 0;
     if (!tune.mm && dir != 0) cand[0] = strided_rows(cls, kind, dims[dir]), cand[1] = 0;
+    bool groups = false;  // plan for lineop_contig_groups
     auto plan_with = [&](int mm) -> int {
         mc3d::PlanRequest rq{cls, kind, bc, dims[dir], dd, alphaF, mm};
         op->plan = mc3d::Plan();
@@ -164,8 +182,9 @@ int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
         // unsigned 32-bit byte offsets and record count, so fields below 4 GiB
         // (536 M points: a 640^3 field and up to about 812^3)
         const bool offsets_ok = npts * 8 < 4294967296L;
+        d.groups = groups ? 1 : 0;
         d.phases = 1;
-        d.phases = mc3d::lineop_fast_phases(d, (size_t)lds_limit);
+        if (!groups) d.phases = mc3d::lineop_fast_phases(d, (size_t)lds_limit);
         op->fast = (p.uniform || p.cshort >= 0) && rows_ok && offsets_ok &&
                    mc3d::lineop_fast_supported(d, (size_t)lds_limit);
         if (tune.family == 2) op->fast = false;
@@ -214,6 +233,17 @@ int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
             return mc3d::fail(rc, err);
         }
     }
+    if (banded && dir == 0 && (bc == MC3D_DIRICHLET || op->plan.cshort >= 0)) {
+        const int mm = grouped_rows(dims[0], op->plan.W, nlines), before = op->plan.MM;
+        groups = mm > 0;
+        if (groups && (plan_with(mm) != MC3D_OK || !op->fast)) {
+            groups = false;
+            if ((rc = plan_with(before)) != MC3D_OK) {
+                delete op;
+                return mc3d::fail(rc, err);
+            }
+        }
+    }
     if (!op->fast && op->plan.MM != 16 && op->plan.MM != 32) {  // the LDS-tiled kernel's chunk sizes
         delete op;
         return mc3d::fail(MC3D_EINVAL, "no kernel for this line operator and chunking");
@@ -246,6 +276,7 @@ int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
     if (op->fast)
         op->kname = std::string(dir != 0 ? (pair ? "lineop_strided_pair<" : p.P > 16 ? "lineop_strided_multi<" : "lineop_strided<")
                                          : pair ? "lineop_contig_pair<"
+                                         : op->dev.groups ? "lineop_contig_groups<"
                                          : op->dev.phases > 1 ? "lineop_contig_ph<" : "lineop_contig<") +
                     std::to_string(p.W) +
                     ", " + std::to_string(p.H) + ", " + std::to_string(p.MM) + ", " + per +

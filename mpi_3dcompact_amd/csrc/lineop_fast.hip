@@ -34,6 +34,8 @@ size_t lineop_fast_lds_bytes(const OpDev &op) {
     }
     if (op.dir == 0) {  // the tile, with the interface values inside it (W = 2) or after it
         const size_t L = contig_lines(op.periodic, op.W, op.cshort >= 0, op.N);
+        if (op.groups)  // one group's lines, or the interface values of all 64
+            return sizeof(double) * std::max((size_t)op.N * (64 / contig_groups(op.MM) + 1), (size_t)64 * (op.NI + 1));
         const int K = L == 64 && op.phases > 1 ? op.phases : 1;
         const size_t rows = K > 1 ? (size_t)((op.P + K - 1) / K) * op.MM + 2 * op.H : (size_t)op.N + 2 * op.H;
         const size_t tile = rows * (L + 1), red = L * (op.NI + 1);
@@ -84,8 +86,10 @@ bool lineop_fast_supported(const OpDev &op, size_t lds_limit) {
     const bool rows = chunk_rows_ok(op.MM) && (op.MM >= 16 || op.periodic) && op.MM >= 2 * h;
     // evenly chunked, or ragged: 16- or 32-row chunks (banded operators 20- and
     // 28-row ones too) and one short second chunk
+    if (op.groups && (op.dir != 0 || w == 0 || op.P > 8 || op.MM < 20 || (op.periodic && op.cshort < 0))) return false;
     const bool chunks = op.cshort < 0 ? op.N == op.P * op.MM
-                                      : (op.MM == 16 || op.MM == 32 || (w > 0 && (op.MM == 20 || op.MM == 28))) &&
+                                      : (op.MM == 16 || op.MM == 32 || (w > 0 && (op.MM == 20 || op.MM == 28)) ||
+                                         (op.groups && op.MM == 24)) &&
                                             op.cshort == 1 && op.P >= 3 &&
                                             op.lshort >= std::max(2 * w, 1) && op.lshort < op.MM &&
                                             op.N == (op.P - 1) * op.MM + op.lshort;

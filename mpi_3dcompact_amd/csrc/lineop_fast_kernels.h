@@ -23,8 +23,9 @@
 // transposed [point][line] layout (row stride lines + 1) with halo rows, so
 // the coalesced fill and the per-lane chunk reads are both free of bank
 // conflicts; each thread issues batches of loads before its LDS writes.
-// 64-line tiles too large for LDS stage their chunks in groups
-// (lineop_contig_ph).
+// Lines of up to eight chunks stage the 64 lines in groups of 32 or 16
+// (lineop_contig_groups); 64-line tiles too large for LDS stage their chunks in
+// groups (lineop_contig_ph).
 //
 // Per chunk: explicit stencil (taps in the reference's summation order, no
 // FMA contraction, so the explicit stage is bitwise that of the reference),
@@ -1124,6 +1125,169 @@ __global__ __launch_bounds__(1024) void lineop_contig_ph(OpDev op, LaunchArgs a)
     }
 }
 
+// x-lines of banded Dirichlet or ragged operators in at most eight chunks (64
+// lines, a wave per chunk, as lineop_contig), staged NG groups of S = 64 / NG
+// lines one after another through one tile of S lines: [point][line], row stride
+// S + 1.  A group's loads are issued one group ahead, so that they are in flight
+// while the lanes of the group before read their windows; the results drain the
+// same way.  The tile of all 64 lines lets one workgroup onto a CU from about 150
+// points on, so its loads, solve and stores follow one another with nothing
+// beside them; a group's tile lets two workgroups of eight waves share the CU
+// (128 registers: 16 waves) and hides one's staging behind the other's solve.
+// Halo rows are not staged: the end chunks of periodic lines read the wrapped
+// rows of the tile (and those of Dirichlet lines too, where the end rows never
+// use them).  Three fields, Pade6 / Penta10 / Compact10 / CommN5Pade, TB/s
+// against the whole tile: 97 points 3.5 / 3.9 / 3.5 / 3.3 -> 4.5 / 4.1 / 4.4 /
+// 4.2, 150 2.9 / 2.5 / 2.9 / 2.5 -> 4.4 / 4.0 / 4.4 / 4.0, 193 3.1 / 2.6 / 3.1 /
+// 2.8 -> 4.0 / 3.7 / 4.0 / 3.8, Dirichlet 160 3.5 / 2.8 / 3.1 / 2.7 -> 4.3 / 4.0 /
+// 4.0 / 3.8, 256 4.3 / 3.4 / 3.4 / 3.1 -> 4.2 / 3.8 / 3.5 / 3.3.  Nine to sixteen
+// chunks gained nothing (one workgroup a CU either way), 64-point lines 0-5%.
+//
+// Two groups up to 20 rows a chunk, four above: the rows of 24 and more leave no
+// registers for half a tile in flight (28-row Compact10, 97 points: 3.9 TB/s with
+// two groups, 4.4 with four; 20-row, 150 points: 4.4 and 4.0).
+__host__ __device__ constexpr int contig_groups(int mm) { return mm <= 20 ? 2 : 4; }
+
+template <int W, int H, int MM, bool PER, bool RG>
+__global__ __launch_bounds__(1024) void lineop_contig_groups(OpDev op, LaunchArgs a) {
+    extern __shared__ double smem[];
+    constexpr int NG = contig_groups(MM), S = 64 / NG, LS = S + 1;
+    constexpr int KG = MM / NG;  // a thread's elements of one group
+    static_assert(MM % NG == 0, "a group's elements per thread");
+    const int N = op.N, P = op.P, NI = op.NI;
+    double *tile = smem;
+    double *red = smem;  // interface values: the tile is dead between the windows and the results
+    const int l = threadIdx.x;
+    const int c = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int tid = threadIdx.y * 64 + l;
+    const int nthr = 64 * P, SN = S * N;  // SN = nthr * KG elements a group (ragged lines: fewer)
+    const int q0 = blockIdx.x * 64;
+    const int rem = a.nlines - q0;
+    // (descriptors end at the field's last line: loads past it return 0, stores are dropped)
+    const unsigned nrec = (unsigned)(rem < 64 ? rem : 64) * (unsigned)N * 8u;
+    const __amdgpu_buffer_rsrc_t rin = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<double *>(a.in[blockIdx.y]) + (long)q0 * N, (short)0, (int)nrec, kRawBufferWord3);
+    const int q = q0 + l;
+    const bool live = q < a.nlines;
+    const int cs = chunk_start<MM, RG>(op, c);
+    const bool short_chunk = RG && c == op.cshort;
+    const int len = short_chunk ? op.lshort : MM;
+    // element tid + k nthr of a group: point (..) % N of line (..) / N
+    const int ll0 = tid / N, p0 = tid - ll0 * N;
+    const int slot0 = p0 * LS + ll0;
+    const int qd = nthr / N, rd = nthr - qd * N;
+    const int step = rd * LS + qd, wrapfix = 1 - N * LS;
+    double v[2][KG];
+    auto load = [&](int g) {
+#pragma unroll
+        for (int k = 0; k < KG; ++k) v[g & 1][k] = bload_nt(rin, (unsigned)(g * SN + tid + k * nthr) * 8u, 0);
+    };
+    double w[MM + 2 * H];
+    load(0);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        if (g > 0) __syncthreads();  // the previous group has read its windows
+        int slot = slot0, pp = p0;
+#pragma unroll
+        for (int k = 0; k < KG; ++k) {
+            if (!RG || tid + k * nthr < SN) tile[slot] = v[g & 1][k];
+            pp += rd;
+            slot += step;
+            if (pp >= N) { pp -= N; slot += wrapfix; }
+        }
+        if (g + 1 < NG) load(g + 1);
+        __syncthreads();
+        if (l / S == g) {
+            const double *col = tile + l % S;
+#pragma unroll
+            for (int j = 0; j < MM + 2 * H; ++j) {
+                int p = cs - H + j;
+                if (j < H) p = p < 0 ? p + N : p;
+                if (j >= MM + H) p = p >= N ? p - N : p;  // (also rows past a short chunk's end, never used)
+                w[j] = col[p * LS];
+            }
+        }
+    }
+    __syncthreads();  // every window is read before the interface values overwrite the tile
+    double y[MM];
+    chunk_rhs<H, MM, PER, has_rows<W, H, PER>()>(op, w, y, c == 0, c == P - 1);
+    chunk_solve<W, MM>(op.lu + (PER && !RG ? 0 : (size_t)c * MM * kLuRec), y);
+    publish<W, MM, RG>(red + l * (NI + 1), c, short_chunk, len, y);
+    __syncthreads();
+    {
+        double s[2 * W];
+        interface_sums<W, PER, RG>(op, c, red + l * (NI + 1), s);
+        const double *sp = op.sp + (PER && !RG ? 0 : (size_t)c * MM * 2 * W);
+        chunk_correct_by<W, MM>([sp](int e) { return sp[e]; }, s, y);
+    }
+    // pass-through lines keep their input (nothing is stored yet)
+    if (live && pass_line(op, 0, q, a.Nx, a.Ny)) {
+#pragma unroll
+        for (int i = 0; i < MM; ++i) y[i] = bload(rin, (unsigned)(l * N + cs + i) * 8u, 0);
+    }
+    const __amdgpu_buffer_rsrc_t rout = __builtin_amdgcn_make_buffer_rsrc(
+        a.out[blockIdx.y] + (long)q0 * N, (short)0, (int)nrec, kRawBufferWord3);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        __syncthreads();  // interface values read (first group) or the previous group's results
+        if (l / S == g) {
+            double *col = tile + l % S;
+#pragma unroll
+            for (int i = 0; i < MM; ++i)
+                if (!RG || i < len) col[(cs + i) * LS] = y[i];
+        }
+        __syncthreads();
+        double r[KG];
+        int slot = slot0, pp = p0;
+#pragma unroll
+        for (int k = 0; k < KG; ++k) {
+            r[k] = !RG || tid + k * nthr < SN ? tile[slot] : 0.0;
+            pp += rd;
+            slot += step;
+            if (pp >= N) { pp -= N; slot += wrapfix; }
+        }
+        if (a.accumulate) {
+#pragma unroll
+            for (int k = 0; k < KG; ++k)
+                if (!RG || tid + k * nthr < SN)
+                    r[k] = bload_nt(rout, (unsigned)(g * SN + tid + k * nthr) * 8u, 0) + r[k];
+        }
+#pragma unroll
+        for (int k = 0; k < KG; ++k)
+            if (!RG || tid + k * nthr < SN) bstore(r[k], rout, (unsigned)(g * SN + tid + k * nthr) * 8u, 0);
+    }
+}
+
+template <int W, int H, int MM, bool PER, bool RG>
+hipError_t launch_groups(const OpDev &op, const LaunchArgs &a, int nfields, hipStream_t st) {
+    dim3 grid((a.nlines + 63) / 64, nfields), block(64, op.P);
+    hipLaunchKernelGGL((lineop_contig_groups<W, H, MM, PER, RG>), grid, block, lineop_fast_lds_bytes(op), st, op, a);
+    return hipGetLastError();
+}
+
+// 20- to 32-row chunks; evenly chunked lines are Dirichlet ones (periodic ones
+// take the 16-line tiles)
+template <int W, int H, bool RG>
+hipError_t launch_groups_mm(const OpDev &op, const LaunchArgs &a, int nfields, hipStream_t st) {
+    if constexpr (RG) {
+        if (op.periodic) switch (op.MM) {
+                case 20: return launch_groups<W, H, 20, true, RG>(op, a, nfields, st);
+                case 24: return launch_groups<W, H, 24, true, RG>(op, a, nfields, st);
+                case 28: return launch_groups<W, H, 28, true, RG>(op, a, nfields, st);
+                case 32: return launch_groups<W, H, 32, true, RG>(op, a, nfields, st);
+                default: return hipErrorInvalidValue;
+            }
+    }
+    if (op.periodic) return hipErrorInvalidValue;
+    switch (op.MM) {
+        case 20: return launch_groups<W, H, 20, false, RG>(op, a, nfields, st);
+        case 24: return launch_groups<W, H, 24, false, RG>(op, a, nfields, st);
+        case 28: return launch_groups<W, H, 28, false, RG>(op, a, nfields, st);
+        case 32: return launch_groups<W, H, 32, false, RG>(op, a, nfields, st);
+        default: return hipErrorInvalidValue;
+    }
+}
+
 template <int W, int H, int MM, bool PER, bool RG>
 hipError_t launch_fast(const OpDev &op, const LaunchArgs &a, int nfields, hipStream_t st) {
     if (op.dir == 0) {
@@ -1183,6 +1347,11 @@ hipError_t launch_fast_bc(const OpDev &op, const LaunchArgs &a, int nfields, hip
 
 template <int W, int H>
 hipError_t launch_fast_mm(const OpDev &op, const LaunchArgs &a, int nfields, hipStream_t st) {
+    if constexpr (W > 0) {
+        if (op.groups)
+            return op.cshort >= 0 ? launch_groups_mm<W, H, true>(op, a, nfields, st)
+                                  : launch_groups_mm<W, H, false>(op, a, nfields, st);
+    }
     if (op.cshort >= 0) {  // ragged lines: 16- or 32-row chunks and one short chunk
         if (op.MM == 16) return launch_fast_bc<W, H, 16, true>(op, a, nfields, st);
         if (op.MM == 32) return launch_fast_bc<W, H, 32, true>(op, a, nfields, st);

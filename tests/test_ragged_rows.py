@@ -92,3 +92,34 @@ def test_even_rows(n, mm, d):
             out = torch.empty_like(fin)
             op.apply([fin], [out])
             assert np.max(np.abs(out.cpu().numpy() - want)) <= 1e-12 * np.max(np.abs(want)), (cls, kind, bc)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [96, 97, 105, 112, 131, 144, 150, 160, 165, 170, 192, 193, 200, 224, 230, 250, 256])
+def test_grouped_x_lines(n):
+    """x-lines of four or eight chunks staged in groups of 32 or 16 lines (1056
+    of them: a last workgroup of 32), Dirichlet and ragged periodic, with
+    pass-through lines and in place, against the oracle at 1e-12."""
+    import torch
+    from mpi_3dcompact_amd.ops import LineOp
+    dims = (n, 33, 32)
+    f = np.random.default_rng(n).normal(size=dims[::-1])
+    fin = torch.from_numpy(f).cuda()
+    for cls, kind, af in OPS:
+        for bc3 in ((0, 0, 0), (1, 0, 0), (1, 1, 1), (0, 1, 1)):
+            bc = bc3[0]
+            if cls == 0 and sum(bc3[1:]):
+                continue
+            dd = 1.0 / n if bc == P.PERIODIC else 1.0 / (n - 1)
+            op = LineOp.deriv(kind, 0, bc, dims, dd) if cls == 0 else LineOp.filter(kind, af, 0, bc3, dims)
+            print(f"n={n} cls={cls} kind={kind} bc3={bc3} {op.kernel()}", flush=True)
+            if bc == P.DIRICHLET:
+                assert op.kernel().startswith("lineop_contig_groups<"), op.kernel()
+            want = P.deriv_field(kind, 0, bc, f, dd) if cls == 0 else P.filter_field(kind, af, 0, list(bc3), f)
+            out = torch.empty_like(fin)
+            op.apply([fin, fin], [out, torch.empty_like(fin)])
+            if cls == 1:
+                same = fin.clone()
+                op.apply([same], [same])
+                assert torch.equal(same, out)
+            assert np.max(np.abs(out.cpu().numpy() - want)) <= 1e-12 * np.max(np.abs(want)), (cls, kind, bc3)
