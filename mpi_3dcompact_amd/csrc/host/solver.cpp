@@ -9,7 +9,6 @@
 #include <cstring>
 #include <fstream>
 
-#include "../dsm.h"
 #include "../stats.h"
 #include "closure.hpp"
 #include "mesh.hpp"
@@ -213,10 +212,36 @@ void DSMSGS::filterQuantity(int n, const double *const *in, double *const *out) 
     }
 }
 
-void DSMSGS::average(int n, const double *const *in, double *const *out) {
-    if (musgsAvgType == Options::LOCAL) filterQuantity(n, in, out);
-    else
-        for (int k = 0; k < n; ++k) doAveraging(in[k], out[k]);
+// The averages of n fields as the kernels after them read them: LOCAL, every
+// point's own value in `local`; line and global averages one value per line or
+// one for the field, in a filter temporary (free between filters); NONE, the
+// fields themselves.
+AvgIndex DSMSGS::average(int n, const double *const *in, double *const *local, const double **out) {
+    const Domain &d = cs->dom;
+    AvgIndex ix{-1, d.gNx, d.gNy};
+    const Options::StatsAvgType t = musgsAvgType;
+    if (t == Options::LOCAL) {
+        filterQuantity(n, in, local);
+        for (int k = 0; k < n; ++k) out[k] = local[k];
+    } else if (t == Options::GLOBAL) {
+        ix.dir = 3;
+        for (int k = 0; k < n; ++k) {
+            out[k] = ftmp_[0] + k;
+            hip_check(launch_mean(in[k], ftmp_[0] + k, cs->cfl_partial, cs->N, cs->st), "global mean");
+        }
+    } else if (t == Options::XI1_AVG || t == Options::XI2_AVG || t == Options::XI3_AVG) {
+        ix.dir = cs->axis_of[t == Options::XI1_AVG ? 0 : t == Options::XI2_AVG ? 1 : 2];
+        const long nl = cs->N / (ix.dir == 0 ? d.gNx : ix.dir == 1 ? d.gNy : d.gNz);
+        double *line[4];
+        for (int k = 0; k < n; ++k) out[k] = line[k] = ftmp_[0] + k * nl;  // n <= 4 of at least 11 lines' room
+        cs->timed("k_xi_average_fields", (double)n, [&] {
+            hip_check(launch_xi_average_fields(in, nullptr, n, ix.dir, d.gNx, d.gNy, d.gNz, cs->st, line),
+                      "line average");
+        });
+    } else {
+        for (int k = 0; k < n; ++k) out[k] = in[k];
+    }
+    return ix;
 }
 
 // src/DSMSGS.hpp:124-343
@@ -229,60 +254,41 @@ void DSMSGS::calcMuSGSTaukk(const double *const dU[3], const double *const dV[3]
     DsmStrainArgs sa{};
     for (int d = 0; d < 3; ++d) { sa.dU[d] = dU[d]; sa.dV[d] = dV[d]; sa.dW[d] = dW[d]; }
     sa.m = cs->msh;
-    sa.rho = rho;
-    for (int k = 0; k < 6; ++k) { sa.S[k] = S[k]; sa.M2[k] = w[1 + k]; }
+    sa.rho = rho; sa.rhoU = rhoU; sa.rhoV = rhoV; sa.rhoW = rhoW;
+    for (int k = 0; k < 6; ++k) { sa.S[k] = S[k]; sa.M2[k] = w[1 + k]; sa.Lt[k] = w[13 + k]; }
     sa.Smag = Smag;
-    cs->timed("k_dsm_strain", 32.0, [&] { hip_check(launch_dsm_strain(sa, N, st), "dsm strain"); });
-    {   // M_ij (work7..12), rho_hat, S_ij hat (work1..6), Smag_hat
-        const double *in[14] = {w[1], w[2], w[3], w[4], w[5], w[6], rho, S[0], S[1], S[2], S[3], S[4], S[5], Smag};
-        double *out[14] = {w[7], w[8], w[9], w[10], w[11], w[12], rho_hat, w[1], w[2], w[3], w[4], w[5], w[6], Smag_hat};
-        filterQuantity(14, in, out);
-    }
-    DsmMLArgs ma{};
-    for (int k = 0; k < 6; ++k) { ma.M[k] = w[7 + k]; ma.S_hat[k] = w[1 + k]; ma.Lt[k] = w[13 + k]; }
-    ma.rho_hat = rho_hat; ma.Smag_hat = Smag_hat;
-    ma.rho = rho; ma.rhoU = rhoU; ma.rhoV = rhoV; ma.rhoW = rhoW;
-    cs->timed("k_dsm_ml", 30.0, [&] { hip_check(launch_dsm_ml(ma, N, st), "dsm M/L"); });
-    {   // L_ij (work1..6), momentum hats
-        const double *in[9] = {w[13], w[14], w[15], w[16], w[17], w[18], rhoU, rhoV, rhoW};
-        double *out[9] = {w[1], w[2], w[3], w[4], w[5], w[6], rhoU_hat, rhoV_hat, rhoW_hat};
-        filterQuantity(9, in, out);
-    }
-    DsmLArgs la{};
-    for (int k = 0; k < 6; ++k) la.L[k] = w[1 + k];
-    la.rhoU_hat = rhoU_hat; la.rhoV_hat = rhoV_hat; la.rhoW_hat = rhoW_hat; la.rho_hat = rho_hat;
-    la.rho = rho; la.Smag = Smag;
-    la.CIdenom = useTaukk ? w[13] : nullptr;
-    cs->timed("k_dsm_l", useTaukk ? 19.0 : 16.0, [&] { hip_check(launch_dsm_l(la, N, st), "dsm L"); });
-    if (useTaukk) {
-        const double *in[1] = {w[13]};
-        double *out[1] = {w[14]};
-        filterQuantity(1, in, out);  // alpha_hat
+    sa.alpha = useTaukk ? w[11] : nullptr;
+    const double metrics = sa.m.J11 ? 9.0 : 0.0;
+    cs->timed("k_dsm_strain", 13.0 + metrics + (useTaukk ? 20.0 : 19.0),
+              [&] { hip_check(launch_dsm_strain(sa, N, st), "dsm strain"); });
+    {   // M_ij (work1..6), L_ij (work13..18), S_ij and alpha in place; rho, |S| and momentum hats
+        const double *in[24] = {w[1], w[2], w[3], w[4], w[5], w[6], S[0], S[1], S[2], S[3], S[4], S[5], w[13], w[14],
+                                w[15], w[16], w[17], w[18], rho, Smag, rhoU, rhoV, rhoW, w[11]};
+        double *out[24] = {w[1], w[2], w[3], w[4], w[5], w[6], S[0], S[1], S[2], S[3], S[4], S[5], w[13], w[14],
+                           w[15], w[16], w[17], w[18], rho_hat, Smag_hat, rhoU_hat, rhoV_hat, rhoW_hat, w[11]};
+        filterQuantity(useTaukk ? 24 : 23, in, out);
     }
     DsmContractArgs ca{};
-    for (int k = 0; k < 6; ++k) { ca.L[k] = w[1 + k]; ca.M[k] = w[7 + k]; }
+    for (int k = 0; k < 6; ++k) { ca.M[k] = w[1 + k]; ca.S_hat[k] = S[k]; ca.L[k] = w[13 + k]; }
+    ca.rhoU_hat = rhoU_hat; ca.rhoV_hat = rhoV_hat; ca.rhoW_hat = rhoW_hat;
     ca.rho_hat = rho_hat; ca.Smag_hat = Smag_hat;
-    ca.alpha_hat = useTaukk ? w[14] : nullptr;
-    ca.CIdenom = w[13];
-    ca.Lkk = w[15]; ca.LijMij = w[17]; ca.MijMij = w[18];
-    cs->timed("k_dsm_contract", useTaukk ? 19.0 : 15.0,
+    ca.alpha_hat = useTaukk ? w[11] : nullptr;
+    ca.CIdenom = w[8];
+    ca.Lkk = w[7]; ca.LijMij = w[9]; ca.MijMij = w[10];
+    cs->timed("k_dsm_contract", useTaukk ? 28.0 : 26.0,
               [&] { hip_check(launch_dsm_contract(ca, N, st), "dsm contractions"); });
-    if (useTaukk) {
-        const double *in[4] = {w[15], w[13], w[17], w[18]};
-        double *out[4] = {w[7], w[8], w[9], w[10]};
-        average(4, in, out);
-    } else {
-        const double *in[2] = {w[17], w[18]};
-        double *out[2] = {w[9], w[10]};
-        average(2, in, out);
-    }
+    const double *avg[4] = {nullptr, nullptr, nullptr, nullptr};  // L_ij M_ij, M_ij M_ij, Lkk, CIdenom
+    const double *in[4] = {w[9], w[10], w[7], w[8]};
+    double *loc[4] = {w[1], w[2], w[3], w[4]};
     DsmMuArgs ua{};
-    ua.rho = rho; ua.Smag = Smag; ua.LijMij_avg = w[9]; ua.MijMij_avg = w[10];
-    ua.Lkk_avg = w[7]; ua.CIdenom_avg = w[8]; ua.J = cs->msh.J;
+    ua.avg = average(useTaukk ? 4 : 2, in, loc, avg);
+    ua.rho = rho; ua.Smag = Smag; ua.LijMij_avg = avg[0]; ua.MijMij_avg = avg[1];
+    ua.Lkk_avg = avg[2]; ua.CIdenom_avg = avg[3]; ua.J = cs->msh.J;
     ua.mu_sgs = mu_sgs; ua.taukk = taukk; ua.C = C; ua.CI = CI;
     ua.use_taukk = useTaukk ? 1 : 0;
     ua.dx = cs->dom.dx; ua.dy = cs->dom.dy; ua.dz = cs->dom.dz;
-    cs->timed("k_dsm_mu", 6.0 + (useTaukk ? 2.0 : 0.0) + (C ? 3.0 : 0.0),
+    const double own = ua.avg.dir < 0 ? 1.0 : 0.0;
+    cs->timed("k_dsm_mu", 4.0 + (useTaukk ? 4.0 : 2.0) * own + (C ? 3.0 : 0.0),
               [&] { hip_check(launch_dsm_mu(ua, N, st), "dsm mu"); });
 }
 
@@ -297,9 +303,12 @@ void DSMSGS::calcKSGS(const double *const dT[3], const double *rho, const double
     na.m = cs->msh;
     na.rho = rho; na.Smag = Smag; na.rhoU = rhoU; na.rhoV = rhoV; na.rhoW = rhoW; na.T = T;
     na.rhoT = w[16];
-    cs->timed("k_dsm_nk", 28.0, [&] { hip_check(launch_dsm_nk(na, N, st), "dsm N/K"); });
+    const double *g[3] = {gT[0], gT[1], gT[2]};
+    if (!na.m.J11)  // the caller's gradient is Cartesian already
+        for (int d = 0; d < 3; ++d) g[d] = dT[d];
+    cs->timed("k_dsm_nk", na.m.J11 ? 28.0 : 16.0, [&] { hip_check(launch_dsm_nk(na, N, st), "dsm N/K"); });
     {   // NRHS (work4..6), KRHS (work10..12), rhoT_hat (work17), gradT hats (work13..15)
-        const double *in[10] = {w[1], w[2], w[3], w[7], w[8], w[9], w[16], gT[0], gT[1], gT[2]};
+        const double *in[10] = {w[1], w[2], w[3], w[7], w[8], w[9], w[16], g[0], g[1], g[2]};
         double *out[10] = {w[4], w[5], w[6], w[10], w[11], w[12], w[17], w[13], w[14], w[15]};
         filterQuantity(10, in, out);
     }
@@ -310,16 +319,15 @@ void DSMSGS::calcKSGS(const double *const dT[3], const double *rho, const double
     nn.rho = rho;
     nn.NiNi = w[4]; nn.NiKi = w[5];
     cs->timed("k_dsm_nn", 18.0, [&] { hip_check(launch_dsm_nn(nn, N, st), "dsm NiNi/NiKi"); });
-    {
-        const double *in[2] = {w[4], w[5]};
-        double *out[2] = {w[6], w[10]};
-        average(2, in, out);
-    }
+    const double *in[2] = {w[4], w[5]};
+    double *loc[2] = {w[6], w[10]};
+    const double *avg[2] = {nullptr, nullptr};
     DsmKArgs ka{};
-    ka.NiNi_avg = w[6]; ka.NiKi_avg = w[10]; ka.rho = rho; ka.Smag = Smag; ka.C = C; ka.J = cs->msh.J;
+    ka.avg = average(2, in, loc, avg);
+    ka.NiNi_avg = avg[0]; ka.NiKi_avg = avg[1]; ka.rho = rho; ka.Smag = Smag; ka.C = C; ka.J = cs->msh.J;
     ka.k_sgs = k_sgs; ka.Prt = Prt;
     ka.cp = cs->ig.cp; ka.dx = cs->dom.dx; ka.dy = cs->dom.dy; ka.dz = cs->dom.dz;
-    cs->timed("k_dsm_ksgs", Prt ? 8.0 : 5.0, [&] { hip_check(launch_dsm_ksgs(ka, N, st), "dsm k_sgs"); });
+    cs->timed("k_dsm_ksgs", (Prt ? 6.0 : 3.0) + (ka.avg.dir < 0 ? 2.0 : 0.0), [&] { hip_check(launch_dsm_ksgs(ka, N, st), "dsm k_sgs"); });
 }
 
 // ---------------------------------------------------------------------------

@@ -14,6 +14,7 @@
 #include <string>
 #include <vector>
 
+#include "../dsm.h"
 #include "../lineop_api.h"
 #include "../pointwise.h"
 #include "mc3d.h"
@@ -221,8 +222,8 @@ class DSMSGS : public AbstractSGS {
     double *ftmp_[16] = {};
     // filterQuantity of n fields: Y into temporaries, Z in place, X into out
     void filterQuantity(int n, const double *const *in, double *const *out);
-    // doAveraging of n fields (batched for LOCAL)
-    void average(int n, const double *const *in, double *const *out);
+    // doAveraging of n <= 4 fields: where the values are, and how a point finds its own
+    AvgIndex average(int n, const double *const *in, double *const *local, const double **out);
 };
 
 // ---------------------------------------------------------------------------

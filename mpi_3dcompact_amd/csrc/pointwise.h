@@ -148,6 +148,8 @@ __device__ __forceinline__ long xi_line_of(long p, int dir, int Nx, int Ny) {
 }
 // per-block {min, max} pairs of phi into partial[2 * nblocks] (getRange)
 hipError_t launch_minmax_partial(const double *phi, double *partial, int nblocks, long n, hipStream_t st);
+// *mean = mean(phi); partial needs cfl_blocks(n) doubles
+hipError_t launch_mean(const double *phi, double *mean, double *partial, long n, hipStream_t st);
 // doAveraging GLOBAL: phiF = mean(phi); partial needs cfl_blocks(n) + 1 doubles
 hipError_t launch_global_mean(const double *phi, double *phiF, double *partial, long n,
                               hipStream_t st);
