@@ -34,18 +34,24 @@ __device__ __forceinline__ f32x4 mfma(const s16x8 &a, const s16x8 &b, const f32x
                                                    c, 0, 0, 0);
 }
 
+// the biases of the four neurons 16t + 4g + r of an output tile
+__device__ __forceinline__ f32x4 bias4(const float *b, int t, int g) {
+    return *reinterpret_cast<const f32x4 *>(b + 16 * t + 4 * g);
+}
+
 constexpr float kG0 = 0.7978845608028654f;  // sqrt(2 / pi)
 constexpr float kG1 = 0.044715f;
 
 // tanh-form GELU 0.5 z (1 + tanh u), u = k0 (z + k1 z^3), written as z s with
 // s = 1 / (1 + exp(-2u)) = (1 + tanh u) / 2 and exp(-2u) = 2^(z (c1 + c2 z^2)),
-// c1 = -2 k0 log2(e), c2 = c1 k1: three FP32 operations, the hardware 2^x and
-// reciprocal (the network's evaluation is bound by these vector operations)
+// c1 = -2 k0 log2(e), c2 = c1 k1: two products and a fused one, the hardware 2^x
+// and reciprocal (the network's evaluation is bound by these vector operations:
+// the biases enter as the products' accumulator for the same reason)
 constexpr float kGc1 = (float)(-2.0 * 0.7978845608028654 * 1.4426950408889634);
 constexpr float kGc2 = (float)(-2.0 * 0.7978845608028654 * 1.4426950408889634 * 0.044715);
 __device__ __forceinline__ float gelu_s(float z) {
     const float z2 = z * z;
-    return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * (kGc1 + kGc2 * z2)));
+    return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * __builtin_fmaf(kGc2, z2, kGc1)));
 }
 __device__ __forceinline__ float gelu(float z) { return z * gelu_s(z); }
 // d/dz, s = gelu_s(z): s + z 2 s (1 - s) k0 (1 + 3 k1 z^2)
@@ -250,18 +256,15 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ P, c
     f32x4 z[3][4];
     s16x8 h[2];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) z[0][t] = mfma(s.w[t][l], x, zero);
+    for (int t = 0; t < 4; ++t) z[0][t] = mfma(s.w[t][l], x, bias4(s.b[0], t, g));
 #pragma unroll
     for (int layer = 0; layer < 3; ++layer) {
         if (layer > 0) {
 #pragma unroll
             for (int t = 0; t < 4; ++t)
-                z[layer][t] = mfma(s.w[8 * layer - 4 + 2 * t + 1][l], h[1], mfma(s.w[8 * layer - 4 + 2 * t][l], h[0], zero));
+                z[layer][t] = mfma(s.w[8 * layer - 4 + 2 * t + 1][l], h[1],
+                                   mfma(s.w[8 * layer - 4 + 2 * t][l], h[0], bias4(s.b[layer], t, g)));
         }
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) z[layer][t][r] = z[layer][t][r] + s.b[layer][16 * t + 4 * g + r];
         train_activate(z[layer], h, s.act[layer], g, smp);
     }
     // ---- output layer, loss, dL/dy (lanes g = 0 hold the two outputs of their sample) ----
@@ -405,126 +408,6 @@ __global__ void k_mlp_adam(float *__restrict__ P, float *__restrict__ m, float *
 }
 
 // ---------------------------------------------------------------------------
-// inference: the network lives in registers as MFMA A operands.  Products are
-// computed transposed, D = W h^T (rows = neurons, columns = 16 samples), so a
-// layer's output D tiles are already the next layer's B operand once the
-// contraction index is permuted: for k-block b, lane group g, element e the
-// neuron is kappa(b, g, e) = 16 (2b + e/4) + 4g + e%4, which is exactly what
-// the lane holds in its output tiles 2b and 2b+1.  No LDS is needed.
-// ---------------------------------------------------------------------------
-struct InferW {
-    s16x8 w1[4];
-    s16x8 w2[4][2], w3[4][2];
-    s16x8 w4[2];
-    float b1[16], b2[16], b3[16];  // [t * 4 + r]: neuron 16t + 4g + r
-    float b4[4];                   // [r]: output 4g + r
-};
-
-__device__ void load_infer(const float *__restrict__ P, InferW &W) {
-    const int l = lane_id(), i = l & 15, g = l >> 4;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int k = 8 * g + e;
-            W.w1[t][e] = k < kMlpIn ? (short)f2bf(P[kMlpOffW1 + (16 * t + i) * kMlpIn + k]) : (short)0;
-        }
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                W.w2[t][b][e] = (short)f2bf(P[kMlpOffW2 + (16 * t + i) * kMlpHid + kappa(b, g, e)]);
-                W.w3[t][b][e] = (short)f2bf(P[kMlpOffW3 + (16 * t + i) * kMlpHid + kappa(b, g, e)]);
-            }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            W.b1[t * 4 + r] = P[kMlpOffB1 + 16 * t + 4 * g + r];
-            W.b2[t * 4 + r] = P[kMlpOffB2 + 16 * t + 4 * g + r];
-            W.b3[t * 4 + r] = P[kMlpOffB3 + 16 * t + 4 * g + r];
-        }
-    }
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-            W.w4[b][e] = i < kMlpOut ? (short)f2bf(P[kMlpOffW4 + i * kMlpHid + kappa(b, g, e)]) : (short)0;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) W.b4[r] = (g == 0 && r < kMlpOut) ? P[kMlpOffB4 + r] : 0.0f;
-}
-
-__device__ __forceinline__ void activate(const f32x4 acc[4], const float *bias, s16x8 h[2]) {
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int t = 2 * b + (e >> 2), r = e & 3;
-            h[b][e] = (short)f2bf(gelu(acc[t][r] + bias[t * 4 + r]));
-        }
-}
-
-// 16 samples: x = layer-1 B operand (lane l, g = 0: features of sample l % 16;
-// other lanes zero).  Returns D of the output layer: lanes with g = 0 hold
-// outputs 0 and 1 of sample l % 16 in elements 0 and 1.
-__device__ __forceinline__ f32x4 infer16(const InferW &W, const s16x8 &x) {
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4 acc[4];
-    s16x8 h[2];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) acc[t] = mfma(W.w1[t], x, zero);
-    activate(acc, W.b1, h);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) acc[t] = mfma(W.w2[t][1], h[1], mfma(W.w2[t][0], h[0], zero));
-    activate(acc, W.b2, h);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) acc[t] = mfma(W.w3[t][1], h[1], mfma(W.w3[t][0], h[0], zero));
-    activate(acc, W.b3, h);
-    f32x4 y = mfma(W.w4[1], h[1], mfma(W.w4[0], h[0], zero));
-#pragma unroll
-    for (int r = 0; r < 4; ++r) y[r] = y[r] + W.b4[r];
-    return y;
-}
-
-// the network on the 64 samples of a wave (lane L: standardised inputs x[7]);
-// returns this lane's two outputs
-__device__ __forceinline__ void infer64(const InferW &W, const float x[kMlpIn], float &y0, float &y1) {
-    const int l = lane_id(), g = l >> 4;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        s16x8 op;
-        const int src = 16 * b + (l & 15);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float v = e < kMlpIn ? __shfl(x[e < kMlpIn ? e : 0], src) : 0.0f;
-            op[e] = (g == 0 && e < kMlpIn) ? (short)f2bf(v) : (short)0;
-        }
-        const f32x4 y = infer16(W, op);
-        const float o0 = __shfl(y[0], l & 15), o1 = __shfl(y[1], l & 15);
-        if (g == b) { y0 = o0; y1 = o1; }
-    }
-}
-
-__global__ __launch_bounds__(256) void k_mlp_infer(const float *__restrict__ P, const float *__restrict__ X,
-                                                   float *__restrict__ Y, long n) {
-    InferW W;
-    load_infer(P, W);
-    const long nwaves = (long)gridDim.x * (blockDim.x >> 6);
-    const long wave = (long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    const long ngroups = (n + 63) / 64;
-    for (long grp = wave; grp < ngroups; grp += nwaves) {
-        const long q = grp * 64 + lane_id();
-        float x[kMlpIn];
-#pragma unroll
-        for (int k = 0; k < kMlpIn; ++k) x[k] = q < n ? X[q * kMlpIn + k] : 0.0f;
-        float y0 = 0.0f, y1 = 0.0f;
-        infer64(W, x, y0, y1);
-        if (q < n) {
-            Y[q * kMlpOut] = y0;
-            Y[q * kMlpOut + 1] = y1;
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
 // per-point features (FP64 -> FP32), shared by the solver closure and sampling
 // ---------------------------------------------------------------------------
 struct GradIn {
@@ -611,21 +494,28 @@ __device__ __forceinline__ void features(const double A[3][3], double vol_J, flo
     f[6] = (float)(log(vol_J) / 3.0);
 }
 
-// The solver's closure keeps the network in LDS and loads a wave's weight
-// operands into registers only around the products of each 64-point group:
-// the FP64 feature phase and the network phase then do not hold their
-// registers at the same time (4 waves per SIMD instead of 1).  Per-lane
+// ---------------------------------------------------------------------------
+// inference: products are computed transposed, D = W h^T (rows = neurons,
+// columns = 16 samples), so a layer's output D tiles are already the next
+// layer's B operand once the contraction index is permuted: for k-block b, lane
+// group g, element e the neuron is kappa(b, g, e) = 16 (2b + e/4) + 4g + e%4,
+// which is exactly what the lane holds in its output tiles 2b and 2b+1.
+//
+// The network stays in LDS and a wave's weight operands are loaded into
+// registers only around the products of each 64-point group: the FP64 feature
+// phase and the network phase then do not hold their registers at the same
+// time (4 waves per SIMD instead of 1).  Per-lane
 // operands are stored [operand][lane] as 16-byte entries (w1 t = 0..3, w2 t,b,
 // w3 t,b, w4 b), biases by neuron.
+// ---------------------------------------------------------------------------
 constexpr int kWOps = 4 + 8 + 8 + 2;
 struct InferLds {
     s16x8 w[kWOps][64];
     float b[3][kMlpHid];
-    float b4[4];
+    float b4[4];  // zero beyond the two outputs
 };
 
-// the per-lane operands of load_infer, written entry by entry by the whole
-// workgroup (no register copy of the network)
+// the operands, written entry by entry by the whole workgroup
 __device__ void stage_infer(const float *__restrict__ P, InferLds &s) {
     for (int idx = threadIdx.x; idx < kWOps * 64 * 8; idx += blockDim.x) {
         const int e = idx & 7, l = (idx >> 3) & 63, op = idx >> 9;
@@ -650,13 +540,13 @@ __device__ void stage_infer(const float *__restrict__ P, InferLds &s) {
     __syncthreads();
 }
 
-__device__ __forceinline__ void activate_lds(const f32x4 acc[4], const float *bias, int g, s16x8 h[2]) {
+__device__ __forceinline__ void activate(const f32x4 z[4], s16x8 h[2]) {
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int t = 2 * b + (e >> 2), r = e & 3;
-            h[b][e] = bf16_bits(gelu(acc[t][r] + bias[16 * t + 4 * g + r]));
+            h[b][e] = bf16_bits(gelu(z[t][r]));
         }
 }
 
@@ -666,7 +556,6 @@ __device__ __forceinline__ void activate_lds(const f32x4 acc[4], const float *bi
 // products.  Returns this lane's two outputs.
 __device__ __forceinline__ void infer64_lds(const InferLds &s, const float x[kMlpIn], float &y0, float &y1) {
     const int l = lane_id(), g = l >> 4;
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     // compiler-only barrier: the operand loads below stay here instead of being
     // hoisted out of the caller's loop (which would keep them live through the
     // feature phase)
@@ -687,8 +576,8 @@ __device__ __forceinline__ void infer64_lds(const InferLds &s, const float x[kMl
             }
             f32x4 acc[4];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) acc[t] = mfma(w[t], op, zero);
-            activate_lds(acc, s.b[0], g, h[b]);
+            for (int t = 0; t < 4; ++t) acc[t] = mfma(w[t], op, bias4(s.b[0], t, g));
+            activate(acc, h[b]);
         }
     }
 #pragma unroll
@@ -700,17 +589,39 @@ __device__ __forceinline__ void infer64_lds(const InferLds &s, const float x[kMl
         for (int b = 0; b < 4; ++b) {
             f32x4 acc[4];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) acc[t] = mfma(w[2 * t + 1], h[b][1], mfma(w[2 * t], h[b][0], zero));
-            activate_lds(acc, s.b[1 + layer], g, h[b]);
+            for (int t = 0; t < 4; ++t)
+                acc[t] = mfma(w[2 * t + 1], h[b][1], mfma(w[2 * t], h[b][0], bias4(s.b[1 + layer], t, g)));
+            activate(acc, h[b]);
         }
     }
     const s16x8 w40 = s.w[20][l], w41 = s.w[21][l];
-    const float b4 = g == 0 ? s.b4[0] : 0.0f, b4b = g == 0 ? s.b4[1] : 0.0f;
+    const f32x4 b4 = *reinterpret_cast<const f32x4 *>(s.b4);  // (the rows of lanes g > 0 are not read)
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-        const f32x4 y = mfma(w41, h[b][1], mfma(w40, h[b][0], zero));
-        const float o0 = __shfl(y[0] + b4, l & 15), o1 = __shfl(y[1] + b4b, l & 15);
+        const f32x4 y = mfma(w41, h[b][1], mfma(w40, h[b][0], b4));
+        const float o0 = __shfl(y[0], l & 15), o1 = __shfl(y[1], l & 15);
         if (g == b) { y0 = o0; y1 = o1; }
+    }
+}
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_mlp_infer(
+    const float *__restrict__ P, const float *__restrict__ X, float *__restrict__ Y, long n) {
+    __shared__ __attribute__((aligned(16))) InferLds net;
+    stage_infer(P, net);
+    const long nwaves = (long)gridDim.x * (blockDim.x >> 6);
+    const long wave = (long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const long ngroups = (n + 63) / 64;
+    for (long grp = wave; grp < ngroups; grp += nwaves) {
+        const long q = grp * 64 + lane_id();
+        float x[kMlpIn];
+#pragma unroll
+        for (int k = 0; k < kMlpIn; ++k) x[k] = q < n ? X[q * kMlpIn + k] : 0.0f;
+        float y0 = 0.0f, y1 = 0.0f;
+        infer64_lds(net, x, y0, y1);
+        if (q < n) {
+            Y[q * kMlpOut] = y0;
+            Y[q * kMlpOut + 1] = y1;
+        }
     }
 }
 
@@ -734,7 +645,7 @@ __global__ __launch_bounds__(256) void k_closure_features(FeatureArgs a, long n)
 }
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_learned_sgs(ClosureArgs a, long n) {
-    __shared__ InferLds net;
+    __shared__ __attribute__((aligned(16))) InferLds net;
     // the input range and standardisation in LDS: read per group instead of
     // held in scalar registers, which spilled to vector-register lanes
     __shared__ MlpScaling sc;
@@ -801,7 +712,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 // the network on lines (LineClosureArgs); the clamp, standardisation and
 // de-standardisation of k_learned_sgs
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_line_closure(LineClosureArgs a) {
-    __shared__ InferLds net;
+    __shared__ __attribute__((aligned(16))) InferLds net;
     stage_infer(a.params, net);
     __shared__ int wcount[4];
     const int l = lane_id(), w = threadIdx.x >> 6;
