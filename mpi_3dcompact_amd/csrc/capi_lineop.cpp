@@ -20,6 +20,7 @@ struct mc3d_lineop {
     int nbatch = 1;         // members stacked along z
     void *dmem = nullptr;
     int device = 0;
+    int lds_limit = 65536;  // bytes a workgroup may have there
     bool fast = false;      // plain applications use the fast kernels
     std::string kname;      // kernel of plain applications
     // transformed-periodic applications run the LDS-tiled kernel, which takes
@@ -136,6 +137,7 @@ int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
         hipDeviceGetAttribute(&lds_limit, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
         return mc3d::fail(MC3D_EHIP, "cannot query the device");
     auto *op = new mc3d_lineop();
+    op->lds_limit = lds_limit;
     std::string err;
     int rc = 0;
     // Chunk rows to try, in order, until one gives a fast kernel: the tuned
@@ -468,5 +470,33 @@ int lineop_launch_accumulate(const mc3d_lineop *op, const double *const *in, dou
                              int nfields, int accumulate, void *stream) {
     const int mode = op->bc == MC3D_PERIODIC ? kModePlainPeriodic : kModePlainDirichlet;
     return apply(op, in, out, nfields, mode, nullptr, accumulate, stream);
+}
+
+int lineop_launch_together(const mc3d_lineop *const ops[3], const double *const *const in[3],
+                           double *const *const out[3], int n, bool &done, void *stream) {
+    done = false;
+    if (n < 1 || 3 * n > kMaxFields) return MC3D_OK;
+    OpSet o{};
+    LaunchArgs a{};
+    const mc3d_lineop *f = ops[0];
+    for (int d = 0; d < 3; ++d) {
+        const mc3d_lineop *op = ops[d];
+        if (!op->fast || op->cls != kDeriv || op->dir != d || op->nbatch != f->nbatch ||
+            std::memcmp(op->dims, f->dims, sizeof(op->dims)))
+            return MC3D_OK;
+        o.op[d] = op->dev;
+        o.nlines[d] = (int)((long)op->dims[0] * op->dims[1] * op->dims[2] * (d == 2 ? 1 : op->nbatch) / op->dims[d]);
+        for (int k = 0; k < n; ++k) {
+            a.in[d * n + k] = in[d][k];
+            a.out[d * n + k] = out[d][k];
+        }
+    }
+    a.Nx = f->dims[0]; a.Ny = f->dims[1]; a.Nz = f->dims[2];
+    a.nbatch = f->nbatch;
+    if (!lineop_together_supported(o, n, f->nbatch, (size_t)f->lds_limit)) return MC3D_OK;
+    const hipError_t e = lineop_launch_together(o, a, n, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(MC3D_EHIP, std::string("line operator launch: ") + hipGetErrorString(e));
+    done = true;
+    return MC3D_OK;
 }
 }  // namespace mc3d

@@ -1058,11 +1058,13 @@ void CurvilinearCSolver::gradientsAndSGS() {
     AbstractDerivatives *dv[3] = {derivX.get(), derivY.get(), derivZ.get()};
     if (les && les->isDSM) {
         // DSM changes p, T, mu and sos before the temperature gradient (:568-594)
-        for (int d = 0; d < 3; ++d) {
-            const double *in[3] = {pr.U, pr.V, pr.W};
-            double *out[3] = {dU[d], dV[d], dW[d]};
-            dv[d]->calc1stDerivFields(3, in, out, false);
-        }
+        const double *in[3] = {pr.U, pr.V, pr.W};
+        double *out[3][3];
+        for (int d = 0; d < 3; ++d) out[d][0] = dU[d], out[d][1] = dV[d], out[d][2] = dW[d];
+        const double *const *ins[3] = {in, in, in};
+        double *const *outs[3] = {out[0], out[1], out[2]};
+        if (!derivsTogether(3, ins, outs))
+            for (int d = 0; d < 3; ++d) dv[d]->calc1stDerivFields(3, in, out[d], false);
         les->calcMuSGSTaukk(dU, dV, dW, s.q[0], s.q[1], s.q[2], s.q[3]);
         timed("k_dsm_taukk_eos", 7.0,
               [&] { hip_check(launch_dsm_taukk_eos(s.q[0], les->taukk, pr, ig, N, st), "dsm tau_kk"); });
@@ -1073,13 +1075,29 @@ void CurvilinearCSolver::gradientsAndSGS() {
         }
         les->calcKSGS(dT, s.q[0], s.q[1], s.q[2], s.q[3], pr.T);
     } else {
-        for (int d = 0; d < 3; ++d) {
-            const double *in[4] = {pr.U, pr.V, pr.W, pr.T};
-            double *out[4] = {dU[d], dV[d], dW[d], dT[d]};
-            dv[d]->calc1stDerivFields(4, in, out, false);
-        }
+        const double *in[4] = {pr.U, pr.V, pr.W, pr.T};
+        double *out[3][4];
+        for (int d = 0; d < 3; ++d) out[d][0] = dU[d], out[d][1] = dV[d], out[d][2] = dW[d], out[d][3] = dT[d];
+        const double *const *ins[3] = {in, in, in};
+        double *const *outs[3] = {out[0], out[1], out[2]};
+        if (!derivsTogether(4, ins, outs))
+            for (int d = 0; d < 3; ++d) dv[d]->calc1stDerivFields(4, in, out[d], false);
         if (les) les->getSGSViscosity(dU, dV, dW, s.q[0]);
     }
+}
+
+bool CurvilinearCSolver::derivsTogether(int n, const double *const *const in[3], double *const *const out[3]) {
+    AbstractDerivatives *dv[3] = {derivX.get(), derivY.get(), derivZ.get()};
+    const mc3d_lineop *ops[3];
+    for (int d = 0; d < 3; ++d) ops[d] = static_cast<LineDerivative *>(dv[d])->op();
+    bool done = false;
+    const int t = timer.begin("lineop_together", 3.0 * n * 16.0 * (double)N);
+    mc3d_check(lineop_launch_together(ops, in, out, n, done, st), "derivatives");
+    if (done)
+        timer.end(t);
+    else
+        timer.cancel(t);
+    return done;
 }
 
 // src/CurvilinearCSolver_Core.cpp:615-773: fluxes and their divergence
@@ -1104,9 +1122,16 @@ void CurvilinearCSolver::flux() {
     const double *p1[5] = {pre[0], pre[1], pre[2], pre[3], pre[4]};
     const double *p2[5] = {pre[5], pre[6], pre[7], pre[8], pre[9]};
     const double *p3[5] = {pre[10], pre[11], pre[12], pre[13], pre[14]};
-    derivX->calc1stDerivFields(5, p1, div, false);
-    derivY->calc1stDerivFields(5, p2, div, true);
-    derivZ->calc1stDerivFields(5, p3, div, true);
+    // (directions launched together write fields of their own, which the stage
+    // update adds in the same order)
+    const double *const *ins[3] = {p1, p2, p3};
+    double *const *outs[3] = {div, tmp, tmp + 5};
+    div_apart_ = derivsTogether(5, ins, outs);
+    if (!div_apart_) {
+        derivX->calc1stDerivFields(5, p1, div, false);
+        derivY->calc1stDerivFields(5, p2, div, true);
+        derivZ->calc1stDerivFields(5, p3, div, true);
+    }
     // the wall rows keep the continuity flux of their own direction alone (:702-760)
     AbstractDerivatives *dv[3] = {derivX.get(), derivY.get(), derivZ.get()};
     for (int d = 0; d < 3; ++d)
@@ -1120,7 +1145,11 @@ void CurvilinearCSolver::flux() {
 void CurvilinearCSolver::stage_update(int op, double a, double b, double c) {
     RkArgs ra{};
     ra.r1 = r1; ra.rk = rk_; ra.k2 = k2; ra.r2 = r2;
-    for (int e = 0; e < 5; ++e) ra.div[e] = div[e];
+    for (int e = 0; e < 5; ++e) {
+        ra.div[e] = div[e];
+        ra.div2[e] = div_apart_ ? tmp[e] : nullptr;
+        ra.div3[e] = div_apart_ ? tmp[5 + e] : nullptr;
+    }
     ra.J = msh.J;
     ra.sc = sc;
     ra.member_pts = dom.members > 1 ? (unsigned)dom.gN : 0u;
@@ -1139,7 +1168,7 @@ void CurvilinearCSolver::stage_update(int op, double a, double b, double c) {
     // last stage) written, plus the registers, plus U V W p T mu written when the
     // update rides along
     static const double reg[9] = {10, 15, 15, 15, 20, 10, 15, 20, 20};
-    timed("k_rhs_rk", 12.0 + (ra.last ? 2.0 : 0.0) + reg[op] + (ra.eos ? 6.0 : 0.0),
+    timed("k_rhs_rk", 12.0 + (div_apart_ ? 10.0 : 0.0) + (ra.last ? 2.0 : 0.0) + reg[op] + (ra.eos ? 6.0 : 0.0),
           [&] { hip_check(launch_rhs_rk(ra, N, st), "stage update"); });
 }
 

@@ -320,6 +320,7 @@ class CurvilinearCSolver {
     // device fields (one slab)
     Metrics msh{};
     double *Jm[10] = {};
+    bool div_apart_ = false;         // eta and zeta divergences in tmp[0..4], tmp[5..9]
     int *planes_vary_ = nullptr;     // Metrics::varies
     double metric_fields_ = 10.0;    // metric fields k_flux and k_vreman stream (0: the first plane)
     bool metrics_exposed_ = false;   // a metric field's address was handed out
@@ -374,6 +375,9 @@ class CurvilinearCSolver {
     // stage methods, in the reference's call order
     void preStep();               // calcDtFromCFL
     void preSubStep();            // preStepDerivatives
+    // derivatives of n fields along x, y, z (in[d] -> out[d]) in one launch; false,
+    // and nothing done, where that does not pay
+    bool derivsTogether(int n, const double *const *const in[3], double *const *const out[3]);
     void gradientsAndSGS();       //   its derivative and SGS part
     void flux();                  //   its flux and divergence part
     void solveEqnSet() {}         // k2 assembly is fused into the RK stage kernel

@@ -34,6 +34,13 @@ void KernelTimer::end(int token) {
     hip_check(hipEventRecord(recs_[token].b, st_), "event record");
 }
 
+void KernelTimer::cancel(int token) {
+    if (token < 0) return;
+    pool_.push_back(recs_.back().a);
+    pool_.push_back(recs_.back().b);
+    recs_.pop_back();
+}
+
 void KernelTimer::collect() {
     if (recs_.empty()) return;
     hip_check(hipStreamSynchronize(st_), "timer synchronize");

@@ -27,6 +27,7 @@ class KernelTimer {
     // returns a token to pass to end(); -1 when disabled
     int begin(const std::string &key, double bytes);
     void end(int token);
+    void cancel(int token);  // the newest record, whose launch was not made
     // synchronises, folds the recorded events into totals, clears the records
     void collect();
     void reset() { collect(); stats_.clear(); }

@@ -11,6 +11,12 @@ namespace mc3d {
 int lineop_launch_accumulate(const mc3d_lineop *op, const double *const *in, double *const *out,
                              int nfields, int accumulate, void *stream);
 
+// derivatives of n fields along x, y and z (in[d] -> out[d]) in one launch where
+// the operators allow it and gain by it: done tells, and nothing is launched
+// otherwise
+int lineop_launch_together(const mc3d_lineop *const ops[3], const double *const *const in[3],
+                           double *const *const out[3], int n, bool &done, void *stream);
+
 // Launch shape of a line operator: rows per chunk (16 or 32; 0 chooses),
 // kernel family (0 chooses: the fast kernels when they take the operator;
 // 1 the fast kernels; 2 the LDS-tiled kernel) and lines per workgroup of the

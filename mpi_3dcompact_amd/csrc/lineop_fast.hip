@@ -109,4 +109,43 @@ hipError_t lineop_launch_fast(const OpDev &op, const LaunchArgs &a, int nfields,
     }
 }
 
+// Waves of one direction's fields up to which the three together pay: past 2.5 a
+// SIMD a direction fills the chip by itself.  RK4 steps, apart -> together: Pade6
+// 32^3 275 -> 182 us, 48^3 318 -> 232, 64^3 (1280 waves) 397 -> 327, four stacked
+// 48^3 (2160) 503 -> 465, two 64^3 (2560) 587 -> 557, four 64^3 (5120) 980 -> 985;
+// Penta10 64^3 417 -> 364, 56^3 429 -> 340.
+constexpr long kTogetherWaves = 2560;
+
+// Waves of a workgroup: more than 4 of the shared kernel's registers (124 Pade6,
+// 189 Penta10 at 16 rows) leave a CU one workgroup: five chunks of 16 at 80^3,
+// Penta10, 638 -> 740 us, seven at 112^3 1430 -> 1730.
+constexpr int kTogetherChunks = 4;
+
+// a 64-line tile of the x-lines with their halo rows, and every direction's
+// interface values (inside the tile for W = 2)
+size_t lineop_together_bytes(const OpSet &o) {
+    const OpDev &x = o.op[0];
+    const size_t tile = (size_t)(x.N + 2 * x.H) * 65, red = (size_t)64 * (x.NI + 1);
+    return sizeof(double) * (x.W == 2 ? std::max(tile, red) : tile + red);
+}
+
+bool lineop_together_supported(const OpSet &o, int nf, int nbatch, size_t lds_limit) {
+    const OpDev &f = o.op[0];
+    if (!((f.W == 1 && f.H == 2) || (f.W == 2 && f.H == 3)) || f.MM < 8 || f.MM > 28 || f.MM % 4) return false;
+    for (int d = 0; d < 3; ++d) {
+        const OpDev &op = o.op[d];
+        // (one kernel instantiation, one workgroup shape)
+        if (op.dir != d || op.W != f.W || op.H != f.H || op.MM != f.MM || op.P != f.P || op.P > kTogetherChunks ||
+            op.N != f.N || op.N != op.P * op.MM || op.cshort >= 0 || !op.periodic || op.nbl + op.nbr != 0)
+            return false;
+        const long blocks = (long)(o.nlines[d] + 63) / 64 * (d == 2 ? nbatch : 1);
+        if (blocks * nf * op.P > kTogetherWaves) return false;
+    }
+    return lineop_together_bytes(o) <= lds_limit / 2;
+}
+
+hipError_t lineop_launch_together(const OpSet &o, const LaunchArgs &a, int nf, hipStream_t st) {
+    return o.op[0].W == 1 ? lineop_launch_together_w1h2(o, a, nf, st) : lineop_launch_together_w2h3(o, a, nf, st);
+}
+
 }  // namespace mc3d

@@ -831,8 +831,16 @@ constexpr int contig_batch() {
     return MM % 16 ? (MM <= 12 ? MM : MM / 2) : 16;
 }
 
-template <int W, int H, int MM, bool PER, bool RG, int L>
-__global__ __launch_bounds__(1024) void lineop_contig(OpDev op, LaunchArgs a) {
+// what a workgroup of a launch of several operators works on: lines 64 bx.. of
+// nlines (z-lines: of member bz)
+struct SetPart {
+    int nlines;
+    unsigned bx, bz;
+};
+
+// body of lineop_contig, and (SET) of a workgroup among several operators'
+template <int W, int H, int MM, bool PER, bool RG, int L, bool SET>
+__device__ __forceinline__ void contig_lines_of(OpDev op, LaunchArgs a, SetPart sp = SetPart{}) {
     extern __shared__ double smem[];
     constexpr int LS = L + 1;  // row stride of the transposed tile
     const int N = op.N, P = op.P, NI = op.NI;
@@ -846,13 +854,13 @@ __global__ __launch_bounds__(1024) void lineop_contig(OpDev op, LaunchArgs a) {
     const int tid = threadIdx.y * L + threadIdx.x;
     const int nthr = L * P;  // L * N = nthr * MM elements (ragged lines: fewer)
     const int LN = L * N;
-    const int q0 = blockIdx.x * L;
+    const int q0 = (SET ? sp.bx : blockIdx.x) * L;
     // The workgroup's lines are consecutive rows of the field: one contiguous
     // block of L * N doubles, element e at point e % N of line e / N.  Buffer
     // descriptors over that block end at the last line of the field, so the
     // loads of a partial last workgroup past it return 0 and its stores there
     // are dropped.
-    const int rem = a.nlines - q0;
+    const int rem = (SET ? sp.nlines : a.nlines) - q0;
     const unsigned nrec = (unsigned)(rem < L ? rem : L) * (unsigned)N * 8u;
     const __amdgpu_buffer_rsrc_t rin = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<double *>(a.in[blockIdx.y]) + (long)q0 * N, (short)0, (int)nrec, kRawBufferWord3);
@@ -911,7 +919,7 @@ __global__ __launch_bounds__(1024) void lineop_contig(OpDev op, LaunchArgs a) {
     const int l = threadIdx.x;
     const int c = L < 64 ? (int)threadIdx.y : __builtin_amdgcn_readfirstlane(threadIdx.y);
     const int q = q0 + l;
-    const bool live = q < a.nlines;
+    const bool live = q < (SET ? sp.nlines : a.nlines);
     const int cs = chunk_start<MM, RG>(op, c);
     const bool short_chunk = RG && c == op.cshort;
     const int len = short_chunk ? op.lshort : MM;
@@ -973,7 +981,7 @@ __global__ __launch_bounds__(1024) void lineop_contig(OpDev op, LaunchArgs a) {
                     if (pp >= N) { pp -= N; slot += wrapfix; }
                 }
             }
-            if (a.accumulate) {
+            if (!SET && a.accumulate) {
                 double o[kB];
 #pragma unroll
                 for (int k = 0; k < kB; ++k) o[k] = bload_nt(rout, (unsigned)(tid + (k0 + k) * nthr) * 8u, 0);
@@ -984,6 +992,82 @@ __global__ __launch_bounds__(1024) void lineop_contig(OpDev op, LaunchArgs a) {
             for (int k = 0; k < kB; ++k) bstore(v[k], rout, (unsigned)(tid + (k0 + k) * nthr) * 8u, 0);
         }
     }
+}
+
+template <int W, int H, int MM, bool PER, bool RG, int L>
+__global__ __launch_bounds__(1024) void lineop_contig(OpDev op, LaunchArgs a) {
+    contig_lines_of<W, H, MM, PER, RG, L, false>(op, a);
+}
+
+// a workgroup's y- or z-lines in lineop_together: lineop_strided for periodic
+// lines in equal chunks.  (Written out, not one function with that kernel: as a
+// call its rows' offsets and stores are scheduled differently, and y-lines of
+// 256^3 take 237 us, five fields, instead of 225.)
+template <int W, int H, int MM>
+__device__ __forceinline__ void strided_set(const OpDev &op, const LaunchArgs &a, SetPart sp) {
+    extern __shared__ double red[];
+    const int l = threadIdx.x;
+    const int c = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int P = op.P, N = op.N, NI = op.NI;
+    const int q = sp.bx * 64 + l;
+    const bool live = q < sp.nlines;
+    const int qq = live ? q : 0;
+    const bool ydir = op.dir == 1;
+    const long points = (long)a.Nx * a.Ny * a.Nz;  // one member's
+    const long member = ydir ? 0 : sp.bz * points;
+    const unsigned fbytes = (unsigned)(points * (ydir ? a.nbatch : 1)) * 8u;
+    const unsigned base = ydir ? (unsigned)(qq / a.Nx) * a.Nx * a.Ny + qq % a.Nx : qq;
+    const unsigned boff = base * 8u, rowb = (unsigned)(ydir ? a.Nx : a.Nx * a.Ny) * 8u;
+    const __amdgpu_buffer_rsrc_t rin = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<double *>(a.in[blockIdx.y]) + member, (short)0, (int)fbytes, kRawBufferWord3);
+    const int s0 = c * MM - H;
+    double w[MM + 2 * H];
+#pragma unroll
+    for (int j = 0; j < MM + 2 * H; ++j) {
+        int p = s0 + j;
+        if (j < H && c == 0) p += N;
+        if (j >= MM + H && c == P - 1) p -= N;
+        w[j] = bload(rin, boff, (unsigned)p * rowb);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    double y[MM];
+    chunk_rhs<H, MM, true, has_rows<W, H, true>()>(op, w, y, c == 0, c == P - 1);
+    chunk_solve<W, MM>(op.lu, y);
+    publish<W, MM, false>(red + l * (NI + 1), c, false, MM, y);
+    __syncthreads();
+    double s[2 * W];
+    interface_sums<W, true, false>(op, c, red + l * (NI + 1), s);
+    const double *corr = op.sp;
+    chunk_correct_by<W, MM>([corr](int e) { return corr[e]; }, s, y);
+    if (!live) return;
+    const __amdgpu_buffer_rsrc_t rout =
+        __builtin_amdgcn_make_buffer_rsrc(a.out[blockIdx.y] + member, (short)0, (int)fbytes, kRawBufferWord3);
+#pragma unroll
+    for (int i = 0; i < MM; ++i) bstore(y[i], rout, boff, (unsigned)(s0 + H + i) * rowb);
+}
+
+// x, y and z derivatives of nf fields each in one launch: launch row blockIdx.y
+// belongs to operator blockIdx.y / nf.  The directions are independent of one
+// another, and small boxes are bound by the number of dependent launches: alone,
+// one direction of a 64^3 box is 64 workgroups a field, and a launch takes 6 us
+// or more however little it does.  Periodic lines in equal chunks; the
+// arithmetic is that of lineop_contig and lineop_strided.  Of stacked members
+// every operator's workgroups count all lines.  A 64^3 RK4 step went from 397
+// to 327 us.
+template <int W, int H, int MM>
+__global__ __launch_bounds__(256) void lineop_together(OpSet o, LaunchArgs a, int nf) {
+    const OpDev &op = o.op[blockIdx.y / nf];
+    SetPart sp{o.nlines[op.dir], blockIdx.x, 0};
+    if (op.dir == 2) {
+        const unsigned blocks = (sp.nlines + 63) / 64;  // of one member
+        sp.bz = blockIdx.x / blocks;
+        sp.bx = blockIdx.x - sp.bz * blocks;
+    }
+    if (sp.bx * 64 >= (unsigned)sp.nlines || sp.bz >= (unsigned)a.nbatch) return;
+    if (op.dir == 0)
+        contig_lines_of<W, H, MM, true, false, 64, true>(op, a, sp);
+    else
+        strided_set<W, H, MM>(op, a, sp);
 }
 
 // x-lines in 64-line tiles (banded Dirichlet or ragged operators, a wave per
@@ -1339,6 +1423,15 @@ hipError_t launch_fast(const OpDev &op, const LaunchArgs &a, int nfields, hipStr
     return hipGetLastError();
 }
 
+template <int W, int H, int MM>
+hipError_t launch_together(const OpSet &o, const LaunchArgs &a, int nf, hipStream_t st) {
+    int blocks = 0;
+    for (int d = 0; d < 3; ++d) blocks = std::max(blocks, (o.nlines[d] + 63) / 64 * (d == 2 ? a.nbatch : 1));
+    hipLaunchKernelGGL((lineop_together<W, H, MM>), dim3(blocks, 3 * nf), dim3(64, o.op[0].P), lineop_together_bytes(o),
+                       st, o, a, nf);
+    return hipGetLastError();
+}
+
 template <int W, int H, int MM, bool RG = false>
 hipError_t launch_fast_bc(const OpDev &op, const LaunchArgs &a, int nfields, hipStream_t st) {
     return op.periodic ? launch_fast<W, H, MM, true, RG>(op, a, nfields, st)
@@ -1384,6 +1477,8 @@ hipError_t lineop_launch_fast_w1h2(const OpDev &op, const LaunchArgs &a, int nfi
 hipError_t lineop_launch_fast_w1h4(const OpDev &op, const LaunchArgs &a, int nfields, hipStream_t st);
 hipError_t lineop_launch_fast_w1h5(const OpDev &op, const LaunchArgs &a, int nfields, hipStream_t st);
 hipError_t lineop_launch_fast_w2h3(const OpDev &op, const LaunchArgs &a, int nfields, hipStream_t st);
+hipError_t lineop_launch_together_w1h2(const OpSet &o, const LaunchArgs &a, int nf, hipStream_t st);
+hipError_t lineop_launch_together_w2h3(const OpSet &o, const LaunchArgs &a, int nf, hipStream_t st);
 hipError_t lineop_launch_fast_w2h5(const OpDev &op, const LaunchArgs &a, int nfields, hipStream_t st);
 
 }  // namespace mc3d

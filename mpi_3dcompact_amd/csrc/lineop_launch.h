@@ -22,6 +22,12 @@ struct LaunchArgs {
     int accumulate;  // out += result instead of out = result
 };
 
+// x, y and z derivative operators launched together (lineop_together)
+struct OpSet {
+    OpDev op[3];
+    int nlines[3];  // as LaunchArgs::nlines
+};
+
 // LDS-tiled kernel, any chunking, all modes (TPB included)
 size_t lineop_lds_bytes(const OpDev &op);
 hipError_t lineop_launch(const OpDev &op, const LaunchArgs &a, int nfields, int mode,
@@ -43,5 +49,10 @@ int lineop_fast_phases(const OpDev &op, size_t lds_limit);
 bool lineop_fast_pair(const OpDev &op);
 int lineop_pair_waves(const OpDev &op);
 hipError_t lineop_launch_fast(const OpDev &op, const LaunchArgs &a, int nfields, hipStream_t st);
+// whether the operators of o, each on nf fields, can share a launch and gain by
+// it, its LDS, and that launch (a.in, a.out: nf entries for each operator)
+bool lineop_together_supported(const OpSet &o, int nf, int nbatch, size_t lds_limit);
+size_t lineop_together_bytes(const OpSet &o);
+hipError_t lineop_launch_together(const OpSet &o, const LaunchArgs &a, int nf, hipStream_t st);
 
 }  // namespace mc3d

@@ -78,6 +78,7 @@ struct RkBc {
 struct RkArgs {
     Cons r1, rk, k2, r2;
     const double *div[5];  // summed flux divergences (cont, mom1..3, engy)
+    const double *div2[5], *div3[5];  // their eta and zeta parts where div holds xi's alone (else null)
     const double *J;
     const StepScalars *sc;  // one per member when member_pts is set: sc[ip / member_pts]
     unsigned member_pts;

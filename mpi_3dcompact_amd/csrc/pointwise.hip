@@ -317,15 +317,21 @@ __global__ __launch_bounds__(kBlock) void k_rhs_rk(RkArgs a, long n) {
 #pragma unroll
         for (int q = 0; q < 5; ++q) z[q] = z0;
     }
+    double div[5];
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {
+        div[q] = ldnt(a.div[q], ip);
+        if (a.div2[q]) div[q] = (div[q] + ldnt(a.div2[q], ip)) + ldnt(a.div3[q], ip);
+    }
     double k2[5];
-    k2[0] = dtJ * (-ldnt(a.div[0], ip) + z[0]);
+    k2[0] = dtJ * (-div[0] + z[0]);
 #pragma unroll
     for (int q = 1; q < 4; ++q) {
-        double v = ldnt(a.k2.q[q], ip) + (-ldnt(a.div[q], ip) + z[q]);
+        double v = ldnt(a.k2.q[q], ip) + (-div[q] + z[q]);
         k2[q] = v * dtJ;
     }
     {
-        double v = -ldnt(a.div[4], ip) + z[4];
+        double v = -div[4] + z[4];
         k2[4] = v * dtJ;
     }
     if (a.bc.active) {  // postStepBCHandling, src/CurvilinearCSolver_BC.cpp:702-842
