@@ -88,10 +88,17 @@ int rotate(int layout, int dir, const int dims[3], const int bc3[3], int vd[3], 
 // points have no such split and keep 32.)  64 points: four chunks of 16 rows
 // instead of two of 32, which leave a 64^3 box 512 waves for 1024 SIMDs
 // (four fields: Pade6 7.7 -> 6.9 us, Penta10 8.6 -> 7.6, Compact10 10.0 -> 7.6).
-int strided_rows(int cls, int kind, int n) {
+// Four chunks beyond 12288 lines no longer pay: the chip is full either way
+// (five fields: 64 points 0.93-0.98 of the time of 32 rows at 9216 lines, 1.05-1.2
+// at 16384; 96 points 0.89-0.92 and up to 1.13).  Compact10's wide window makes six
+// chunks of 24 rows slower than nine of 16 up to 24576 lines (1.04-1.06; 0.95 at
+// 36864 and more), where Penta10's take 0.79-0.87.
+int strided_rows(int cls, int kind, int n, long nlines) {
     const bool banded = cls == mc3d::kDeriv ? kind != MC3D_CD2 : kind != MC3D_COMMN5EXP;
     if (!banded || n % 16 != 0) return 0;
+    if (n <= 96 && nlines > 12288) return 0;
     if (n / 32 == 2) return n % 32 ? 0 : 16;
+    if (n == 6 * 24 && cls == mc3d::kFilter && kind == MC3D_COMPACT10 && nlines <= 24576) return 0;
     for (int mm : {24, 28, 20}) {
         const int P = n / mm;
         if (n % mm == 0 && (P == 6 || P == 8 || P == 12 || P == 16 || (P == 4 && mm == 24))) return mm;
@@ -104,10 +111,16 @@ int strided_rows(int cls, int kind, int n) {
 // chunks, whose waves spread evenly over a CU's SIMDs (the fewest rows that give
 // at most so many; 144 points: eight chunks of 20 rows 3.6-4.0 TB/s, six of 24
 // 2.9-3.4).  113 to 128 points are eight 16-row chunks, which the whole tile serves
-// as well.  Fewer than 1024 lines leave most of the chip idle either way and keep
-// the whole tile, as do shorter lines, of which several tiles fit a CU.
+// as well.  The second workgroup of a CU is the gain, so a launch has to have one:
+// with up to 16384 lines a field is 256 workgroups, and one field of 160 to 256
+// points takes 1.0-1.5 times the whole tile's time (four fields 1.0-1.4 up to 4096
+// lines, 0.7-0.9 from 6144 on); at 17408 lines 0.72-0.90.  Whole tiles of up to 112
+// points fit a CU three at a time and win up to 32768 lines of one field (1.06-1.3;
+// 0.75-1.02 at 49152).  Unevenly chunked lines below 160 points gain at any count
+// (129-158 points 0.86-1.02 at 4096 lines, 0.59-1.02 beyond).
 int grouped_rows(int n, int W, long nlines) {
-    if (n < 96 || n > 256 || nlines < 1024 || (n > 112 && n <= 128)) return 0;
+    if (n < 96 || n > 256 || (n > 112 && n <= 128)) return 0;
+    if (nlines < (n <= 112 ? 49152 : n < 160 && n % 16 ? 4096 : 16385)) return 0;
     const int chunks = n <= 112 ? 4 : 8;
     for (int mm : {20, 24, 28, 32}) {
         const int P = (n + mm - 1) / mm, rem = n - (P - 1) * mm;
@@ -149,9 +162,10 @@ int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
     // which also serves lines too long for 16-row chunks in one workgroup;
     // for y- and z-lines strided_rows first.
     // When none is fast, 16-row chunks for the LDS-tiled kernel.
+    const long nlines = npts / nbatch / dims[dir];  // one member's: a stacked box takes its members' kernels
     int cand[2] = {tune.mm, -1};
     if (!tune.mm && dir == 0 && dims[0] % 16 == 0) cand[0] = 16, cand[1] = 0;
-    if (!tune.mm && dir != 0) cand[0] = strided_rows(cls, kind, dims[dir]), cand[1] = 0;
+    if (!tune.mm && dir != 0) cand[0] = strided_rows(cls, kind, dims[dir], nlines), cand[1] = 0;
     bool groups = false;  // plan for lineop_contig_groups
     auto plan_with = [&](int mm) -> int {
         mc3d::PlanRequest rq{cls, kind, bc, dims[dir], dd, alphaF, mm};
@@ -222,7 +236,6 @@ int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
     // Fewer lines keep the plan's own choice: one field of so small a box is
     // launch latency either way (272 Penta10 lines of 131 points 21 -> 11 us).
     const bool banded = op->plan.W > 0 && !tune.mm && tune.family != 2;
-    const long nlines = npts / nbatch / dims[dir];  // one member's: a stacked box takes its members' kernels
     const int planned = op->plan.MM;
     const bool rescue = !op->fast, mid = op->fast && dir != 0 && op->plan.cshort >= 0 && op->plan.MM == 32 && dims[dir] <= 320;
     if (banded && nlines >= 512 && (rescue || mid)) {

@@ -87,7 +87,8 @@ def test_even_rows(n, mm, d):
             bc3 = [0, 0, 0]
             bc3[d] = bc
             op = LineOp.deriv(kind, d, bc, dims, dd) if cls == 0 else LineOp.filter(kind, af, d, bc3, dims)
-            assert f", {mm}, " in op.kernel() and op.kernel().startswith("lineop_strided<"), op.kernel()
+            rows = 16 if n == 144 and (cls, kind) == (1, P.COMPACT10) else mm
+            assert f", {rows}, " in op.kernel() and op.kernel().startswith("lineop_strided<"), op.kernel()
             want = P.deriv_field(kind, d, bc, f, dd) if cls == 0 else P.filter_field(kind, af, d, bc3, f)
             out = torch.empty_like(fin)
             op.apply([fin], [out])
@@ -97,14 +98,16 @@ def test_even_rows(n, mm, d):
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [96, 97, 105, 112, 131, 144, 150, 160, 165, 170, 192, 193, 200, 224, 230, 250, 256])
 def test_grouped_x_lines(n):
-    """x-lines of four or eight chunks staged in groups of 32 or 16 lines (1056
-    of them: a last workgroup of 32), Dirichlet and ragged periodic, with
-    pass-through lines and in place, against the oracle at 1e-12."""
+    """x-lines of four or eight chunks staged in groups of 32 or 16 lines (17424
+    or 49632 of them: a last workgroup of 16 or 32), Dirichlet and ragged periodic,
+    with pass-through lines and in place, the first and last eight z-planes
+    against the oracle at 1e-12."""
     import torch
     from mpi_3dcompact_amd.ops import LineOp
-    dims = (n, 33, 32)
+    dims = (n, 33, 528 if n > 112 else 1504)
     f = np.random.default_rng(n).normal(size=dims[::-1])
     fin = torch.from_numpy(f).cuda()
+    ends = np.r_[0:8, dims[2] - 8:dims[2]]
     for cls, kind, af in OPS:
         for bc3 in ((0, 0, 0), (1, 0, 0), (1, 1, 1), (0, 1, 1)):
             bc = bc3[0]
@@ -115,11 +118,30 @@ def test_grouped_x_lines(n):
             print(f"n={n} cls={cls} kind={kind} bc3={bc3} {op.kernel()}", flush=True)
             if bc == P.DIRICHLET:
                 assert op.kernel().startswith("lineop_contig_groups<"), op.kernel()
-            want = P.deriv_field(kind, 0, bc, f, dd) if cls == 0 else P.filter_field(kind, af, 0, list(bc3), f)
+            sub = np.ascontiguousarray(f[ends])
+            want = P.deriv_field(kind, 0, bc, sub, dd) if cls == 0 else P.filter_field(kind, af, 0, list(bc3), sub)
             out = torch.empty_like(fin)
             op.apply([fin, fin], [out, torch.empty_like(fin)])
             if cls == 1:
                 same = fin.clone()
                 op.apply([same], [same])
                 assert torch.equal(same, out)
-            assert np.max(np.abs(out.cpu().numpy() - want)) <= 1e-12 * np.max(np.abs(want)), (cls, kind, bc3)
+            assert np.max(np.abs(out.cpu().numpy()[ends] - want)) <= 1e-12 * np.max(np.abs(want)), (cls, kind, bc3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,few,many", [(160, 16384, 16385), (256, 16384, 16385), (112, 49151, 49152), (150, 4095, 4096)])
+def test_grouped_line_counts(n, few, many):
+    """Too few x-lines for two workgroups a CU keep the whole tile."""
+    from mpi_3dcompact_amd.ops import LineOp
+    assert LineOp.deriv(P.PENTA10, 0, P.DIRICHLET, (n, few, 1), 1.0).kernel().startswith("lineop_contig<")
+    assert LineOp.deriv(P.PENTA10, 0, P.DIRICHLET, (n, many, 1), 1.0).kernel().startswith("lineop_contig_groups<")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,rows", [(64, 16), (96, 24)])
+def test_four_chunk_line_counts(n, rows):
+    """Four chunks of y/z-lines up to 12288 lines only."""
+    from mpi_3dcompact_amd.ops import LineOp
+    assert f", {rows}, " in LineOp.deriv(P.PENTA10, 2, P.PERIODIC, (128, 96, n), 1.0).kernel()
+    assert ", 32, " in LineOp.deriv(P.PENTA10, 2, P.PERIODIC, (128, 97, n), 1.0).kernel()
