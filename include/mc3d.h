@@ -431,8 +431,8 @@ int mc3d_dump_write(const char *path, int timestep, double time, const int dims[
 /* Diagnostic (no counterpart in the reference): builds, on the host only,
  * the partition tables an operator would upload, for verification of the
  * factorisation without a GPU.  cls 0 = derivative (kind = scheme), 1 = filter
- * (kind = filter kind); mm = rows per chunk (16 or 32, 0 = the choice the
- * operators make).  sizes[11] receives {N, W, H, P, NI, nbl, nbr, int_off, MM,
+ * (kind = filter kind); mm = rows per chunk (8, 12, .. 32; 0 = the length's
+ * own choice, which an operator may replace: mc3d_plan_kernel).  sizes[11] receives {N, W, H, P, NI, nbl, nbr, int_off, MM,
  * dense_ok, gb} (gb: the interface band in chunks the fast kernels use, G
  * blocks farther from a chunk being below 1e-17 of its largest); each
  * non-NULL table pointer must have room for the sizes
@@ -442,6 +442,14 @@ int mc3d_dump_write(const char *path, int timestep, double time, const int dims[
 int mc3d_plan_tables(int cls, int kind, int bc, int n, double dd, double alphaF, int mm,
                      int sizes[11], double *lu, double *sp, double *G, double *rows,
                      double *drows, double *interior, int *cstart, int *clen);
+
+/* Diagnostic (no counterpart in the reference): the name (mc3d_lineop_kernel)
+ * of the kernel that plain applications of an operator in the MC3D_XPENCIL
+ * layout run on a device whose workgroups may have lds_limit bytes of LDS,
+ * chosen on the host without a GPU.  cls and kind as above; MC3D_EINVAL and
+ * MC3D_ENUMERIC where creating the operator gives them. */
+int mc3d_plan_kernel(int cls, int kind, int dir, const int bc3[3], const int dims[3], double dd, double alphaF,
+                     int lds_limit, char *name, int len);
 
 /* ---------------------------------------------------------------------------
  * Ensembles (no counterpart in the reference, which runs one box per job):

@@ -4,6 +4,7 @@
 #include <cmath>
 #include <cstring>
 #include <string>
+#include <vector>
 
 #include "capi_common.h"
 #include "lineop_api.h"
@@ -76,6 +77,9 @@ int rotate(int layout, int dir, const int dims[3], const int bc3[3], int vd[3], 
     return MC3D_OK;
 }
 
+// an operator with an implicit part (W > 0)
+bool banded(int cls, int kind) { return cls == mc3d::kDeriv ? kind != MC3D_CD2 : kind != MC3D_COMMN5EXP; }
+
 // Rows per chunk of evenly chunked y- and z-lines of banded operators, or 0 for
 // the plan's own choice (32 or 16 rows).  A workgroup is one wave per chunk, so
 // the chunk count sets how well workgroups pack into a CU's wave slots: 6, 8,
@@ -94,8 +98,7 @@ int rotate(int layout, int dir, const int dims[3], const int bc3[3], int vd[3], 
 // chunks of 24 rows slower than nine of 16 up to 24576 lines (1.04-1.06; 0.95 at
 // 36864 and more), where Penta10's take 0.79-0.87.
 int strided_rows(int cls, int kind, int n, long nlines) {
-    const bool banded = cls == mc3d::kDeriv ? kind != MC3D_CD2 : kind != MC3D_COMMN5EXP;
-    if (!banded || n % 16 != 0) return 0;
+    if (!banded(cls, kind) || n % 16 != 0) return 0;
     if (n <= 96 && nlines > 12288) return 0;
     if (n / 32 == 2) return n % 32 ? 0 : 16;
     if (n == 6 * 24 && cls == mc3d::kFilter && kind == MC3D_COMPACT10 && nlines <= 24576) return 0;
@@ -129,10 +132,7 @@ int grouped_rows(int n, int W, long nlines) {
     return 0;
 }
 
-int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[3], double dd,
-           double alphaF, int nbatch, const mc3d::LineTune &tune, mc3d_lineop **out) {
-    if (!out) return mc3d::fail(MC3D_EINVAL, "null output handle");
-    *out = nullptr;
+int check_request(int cls, int dir, int bc, const int dims[3], double dd, int nbatch, const mc3d::LineTune &tune) {
     if (!dims || dims[0] <= 0 || dims[1] <= 0 || dims[2] <= 0)
         return mc3d::fail(MC3D_EINVAL, "dims must be positive");
     if (dir < 0 || dir > 2) return mc3d::fail(MC3D_EINVAL, "dir must be 0, 1 or 2");
@@ -145,31 +145,21 @@ int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
     if (tune.family < 0 || tune.family > 2) return mc3d::fail(MC3D_EINVAL, "bad kernel family");
     if (tune.lines < 0 || (tune.lines & (tune.lines - 1)) != 0)
         return mc3d::fail(MC3D_EINVAL, "lines per workgroup must be a power of two");
-    int dev = 0, lds_limit = 65536;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&lds_limit, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
-        return mc3d::fail(MC3D_EHIP, "cannot query the device");
-    auto *op = new mc3d_lineop();
+    return MC3D_OK;
+}
+
+// Plan, kernel and launch shape of an operator (all but its device tables), for a
+// device whose workgroups may have lds_limit bytes of LDS.
+int choose(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[3], double dd, double alphaF,
+           int nbatch, const mc3d::LineTune &tune, int lds_limit, mc3d_lineop *op) {
+    const long npts = (long)dims[0] * dims[1] * dims[2] * nbatch;
     op->lds_limit = lds_limit;
     std::string err;
-    int rc = 0;
-    // Chunk rows to try, in order, until one gives a fast kernel: the tuned
-    // value alone; else for x-lines that split into 16-row chunks 16 first
-    // (contiguous lines are staged whole in LDS, which bounds the waves per
-    // CU; 16-row chunks double them, and measured faster for every x operator:
-    // the Penta10 derivative of 256-point lines inside the LES step 3.3 ->
-    // 2.9 ms), then the plan's own choice (32 rows or an even 8..28-row split),
-    // which also serves lines too long for 16-row chunks in one workgroup;
-    // for y- and z-lines strided_rows first.
-    // When none is fast, 16-row chunks for the LDS-tiled kernel.
-    const long nlines = npts / nbatch / dims[dir];  // one member's: a stacked box takes its members' kernels
-    int cand[2] = {tune.mm, -1};
-    if (!tune.mm && dir == 0 && dims[0] % 16 == 0) cand[0] = 16, cand[1] = 0;
-    if (!tune.mm && dir != 0) cand[0] = strided_rows(cls, kind, dims[dir], nlines), cand[1] = 0;
     bool groups = false;  // plan for lineop_contig_groups
     auto plan_with = [&](int mm) -> int {
         mc3d::PlanRequest rq{cls, kind, bc, dims[dir], dd, alphaF, mm};
         op->plan = mc3d::Plan();
+        op->fast = false;
         int r = mc3d::build_plan(rq, op->plan, err);
         if (r) return r;
         const mc3d::Plan &p = op->plan;
@@ -206,83 +196,98 @@ int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
         if (tune.family == 2) op->fast = false;
         return MC3D_OK;
     };
-    for (int mm : cand) {
-        if (mm < 0) break;
-        rc = plan_with(mm);
-        if (rc) {
-            delete op;
-            return mc3d::fail(rc, err);
+    // Rows per chunk to try, in order, until one gives a fast kernel: the tuned
+    // value alone; else for x-lines that split into 16-row chunks 16 first
+    // (contiguous lines are staged whole in LDS, which bounds the waves per
+    // CU; 16-row chunks double them, and measured faster for every x operator:
+    // the Penta10 derivative of 256-point lines inside the LES step 3.3 ->
+    // 2.9 ms), then the plan's own choice (32 rows or an even 8..28-row split),
+    // which also serves lines too long for 16-row chunks in one workgroup;
+    // for y- and z-lines strided_rows first.  Then 16.
+    // A split whose last chunk is too short for its interface blocks is passed
+    // over (257 points in 16-row chunks); a singular operator is not.  Where no
+    // split is fast the LDS-tiled kernel takes the line in 16-row chunks, or in
+    // 32-row ones where 16 do not split it.
+    const long nlines = npts / nbatch / dims[dir];  // one member's: a stacked box takes its members' kernels
+    int rc = MC3D_OK;       // why the first split failed
+    std::string why;
+    bool singular = false;
+    mc3d::Plan tiled;       // for the LDS-tiled kernel
+    mc3d::OpDev tiled_dev{};
+    auto fast_with = [&](int mm) {
+        const int r = plan_with(mm);
+        if (r) {
+            if (!rc) rc = r, why = err;
+            singular = singular || r != MC3D_EINVAL;
+            return false;
         }
-        if (op->fast) break;
+        if (!op->fast && (op->plan.MM == 16 || (op->plan.MM == 32 && !tiled.P))) tiled = op->plan, tiled_dev = op->dev;
+        return op->fast;
+    };
+    std::vector<int> cand{tune.mm};
+    if (!tune.mm) {
+        const int first = dir == 0 ? (dims[0] % 16 == 0 ? 16 : 0) : strided_rows(cls, kind, dims[dir], nlines);
+        cand = first ? std::vector<int>{first, 0, 16} : std::vector<int>{0, 16};
     }
-    if (!op->fast && !tune.mm && op->plan.MM != 16) {
-        rc = plan_with(16);
-        if (rc) {
-            delete op;
-            return mc3d::fail(rc, err);
-        }
+    bool found = false, tried16 = false;
+    for (int mm : cand) {
+        if (found || singular || (mm == 16 && tried16)) continue;
+        found = fast_with(mm);
+        tried16 = tried16 || op->plan.MM == 16;
     }
     // Banded ragged lines of 512 lines or more, in 20-row chunks (28 where those
     // leave the short chunk fewer than 2W rows) and one short chunk:
     //  - lines whose remainder over 16 (32) rows is too short for its interface
-    //    blocks (65, 129, 193 points, say), which only the LDS-tiled kernel
-    //    took: 129-point Penta10 y in a 160 x 129 x 144 box, four fields,
-    //    305 -> 42 us (0.62 -> 4.6 TB/s; 28 rows 50 us), Compact8 138 -> 48;
-    //    193-point x 1450 -> 399 and 748 -> 351 us (three fields);
+    //    blocks (65, 129, 193, 257 points, say), which only the LDS-tiled kernel
+    //    takes otherwise: 129-point Penta10 y in a 160 x 129 x 144 box, four
+    //    fields, 305 -> 42 us (0.62 -> 4.6 TB/s; 28 rows 50 us), Compact8 138 ->
+    //    48; 193-point x 1450 -> 399 and 748 -> 351 us (three fields);
     //  - y- and z-lines of 257 to 320 points, at most 16 chunks: 310-point
     //    Penta10 z 231 -> 200 us against 32-row chunks (4.0 -> 4.6 TB/s), Compact8
     //    210 -> 189 (28 rows 199).  Shorter ragged y- and z-lines keep 16 rows
     //    (165 points: 67 against 70 us), longer ones 32.
-    // Fewer lines keep the plan's own choice: one field of so small a box is
-    // launch latency either way (272 Penta10 lines of 131 points 21 -> 11 us).
-    const bool banded = op->plan.W > 0 && !tune.mm && tune.family != 2;
-    const int planned = op->plan.MM;
-    const bool rescue = !op->fast, mid = op->fast && dir != 0 && op->plan.cshort >= 0 && op->plan.MM == 32 && dims[dir] <= 320;
-    if (banded && nlines >= 512 && (rescue || mid)) {
-        for (int mm : {20, 28}) {
-            if (dims[dir] % mm == 0 || (mid && mm == 28)) continue;
-            if (plan_with(mm) == MC3D_OK && op->fast) break;
-        }
-        if (!op->fast && (rc = plan_with(planned)) != MC3D_OK) {
-            delete op;
-            return mc3d::fail(rc, err);
-        }
+    // Fewer lines stay on the LDS-tiled kernel, although 20 rows would be faster
+    // there too (272 Penta10 lines of 131 points 21 -> 11 us): a launch of so
+    // small a box is mostly latency.
+    const bool auto_rows = banded(cls, kind) && !tune.mm && tune.family != 2;
+    const bool mid = found && dir != 0 && op->plan.cshort >= 0 && op->plan.MM == 32 && dims[dir] <= 320;
+    if (auto_rows && !singular && nlines >= 512 && (!found || mid)) {
+        const mc3d::Plan p32 = mid ? op->plan : mc3d::Plan();
+        const mc3d::OpDev d32 = op->dev;
+        found = false;
+        for (int mm : {20, 28})
+            if (!found && dims[dir] % mm != 0 && !(mid && mm == 28)) found = plan_with(mm) == MC3D_OK && op->fast;
+        if (!found && mid) op->plan = p32, op->dev = d32, op->fast = found = true;
     }
-    if (banded && dir == 0 && (bc == MC3D_DIRICHLET || op->plan.cshort >= 0)) {
-        const int mm = grouped_rows(dims[0], op->plan.W, nlines), before = op->plan.MM;
-        groups = mm > 0;
-        if (groups && (plan_with(mm) != MC3D_OK || !op->fast)) {
-            groups = false;
-            if ((rc = plan_with(before)) != MC3D_OK) {
-                delete op;
-                return mc3d::fail(rc, err);
-            }
-        }
+    // few lines that 16-row chunks leave too short a remainder (241 points)
+    if (!found && !singular && !tune.mm && !tiled.P) found = fast_with(32);
+    if (!found) {
+        if (!tiled.P) return mc3d::fail(rc ? rc : MC3D_EINVAL, rc ? why : "no kernel for this line operator and chunking");
+        op->plan = tiled;
+        op->dev = tiled_dev;
+        op->fast = false;
     }
-    if (!op->fast && op->plan.MM != 16 && op->plan.MM != 32) {  // the LDS-tiled kernel's chunk sizes
-        delete op;
-        return mc3d::fail(MC3D_EINVAL, "no kernel for this line operator and chunking");
+    if (auto_rows && dir == 0 && (bc == MC3D_DIRICHLET || op->plan.cshort >= 0)) {
+        const int mm = grouped_rows(dims[0], op->plan.W, nlines);
+        if (mm > 0) {
+            const mc3d::Plan whole = op->plan;
+            const mc3d::OpDev dev = op->dev;
+            const bool fast = op->fast;
+            groups = true;
+            if (plan_with(mm) != MC3D_OK || !op->fast) op->plan = whole, op->dev = dev, op->fast = fast;
+        }
     }
     const mc3d::Plan &p = op->plan;
-    if (tune.family == 1 && !op->fast) {
-        delete op;
+    if (tune.family == 1 && !op->fast)
         return mc3d::fail(MC3D_EINVAL, "the fast kernels do not take this line operator and chunking");
-    }
-    if (nbatch > 1 && (op->dev.passA || op->dev.passB)) {
-        delete op;
+    if (nbatch > 1 && (op->dev.passA || op->dev.passB))
         return mc3d::fail(MC3D_EINVAL, "stacked members need periodic lines in the other directions");
-    }
     if (tune.lines) {
         op->dev.L = op->plan.L = tune.lines;
-        if (tune.lines * p.P > 256) {
-            delete op;
+        if (tune.lines * p.P > 256)
             return mc3d::fail(MC3D_EINVAL, "lines per workgroup times chunks exceeds 256 lanes");
-        }
     }
-    if (mc3d::lineop_lds_bytes(op->dev) > 65536) {
-        delete op;
-        return mc3d::fail(MC3D_EINVAL, "line too long for the LDS tile");
-    }
+    if (mc3d::lineop_lds_bytes(op->dev) > 65536) return mc3d::fail(MC3D_EINVAL, "line too long for the LDS tile");
     op->cls = cls; op->kind = kind; op->dir = dir; op->bc = bc;
     op->nbatch = nbatch;
     std::memcpy(op->dims, dims, sizeof(op->dims));
@@ -299,6 +304,26 @@ int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
     else
         op->kname = "lineop_kernel<" + std::to_string(p.W) + ", " + std::to_string(dir) + ", " +
                     std::to_string(bc == MC3D_PERIODIC ? 0 : 1) + ", " + std::to_string(p.MM) + ">";
+    return MC3D_OK;
+}
+
+int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[3], double dd,
+           double alphaF, int nbatch, const mc3d::LineTune &tune, mc3d_lineop **out) {
+    if (!out) return mc3d::fail(MC3D_EINVAL, "null output handle");
+    *out = nullptr;
+    int rc = check_request(cls, dir, bc, dims, dd, nbatch, tune);
+    if (rc) return rc;
+    int dev = 0, lds_limit = 65536;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&lds_limit, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
+        return mc3d::fail(MC3D_EHIP, "cannot query the device");
+    auto *op = new mc3d_lineop();
+    rc = choose(cls, kind, dir, bc, bc3, dims, dd, alphaF, nbatch, tune, lds_limit, op);
+    if (rc) {
+        delete op;
+        return rc;
+    }
+    const mc3d::Plan &p = op->plan;
     rc = upload(op);
     if (rc) {
         if (op->dmem) (void)hipFree(op->dmem);
@@ -450,6 +475,21 @@ int mc3d_plan_tables(int cls, int kind, int bc, int n, double dd, double alphaF,
     }
     if (cstart) std::memcpy(cstart, p.cstart.data(), sizeof(int) * p.P);
     if (clen) std::memcpy(clen, p.clen.data(), sizeof(int) * p.P);
+    return MC3D_OK;
+}
+
+int mc3d_plan_kernel(int cls, int kind, int dir, const int bc3[3], const int dims[3], double dd, double alphaF,
+                     int lds_limit, char *name, int len) {
+    if (!bc3 || !name || len < 1) return mc3d::fail(MC3D_EINVAL, "null argument");
+    if (dir < 0 || dir > 2) return mc3d::fail(MC3D_EINVAL, "dir must be 0, 1 or 2");
+    const mc3d::LineTune t{};
+    int rc = check_request(cls, dir, bc3[dir], dims, dd, 1, t);
+    if (rc) return rc;
+    mc3d_lineop op;
+    rc = choose(cls, kind, dir, bc3[dir], cls == mc3d::kFilter ? bc3 : nullptr, dims, dd, alphaF, 1, t, lds_limit, &op);
+    if (rc) return rc;
+    if ((int)op.kname.size() >= len) return mc3d::fail(MC3D_EINVAL, "name buffer too small");
+    std::memcpy(name, op.kname.c_str(), op.kname.size() + 1);
     return MC3D_OK;
 }
 

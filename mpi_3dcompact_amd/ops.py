@@ -104,6 +104,14 @@ class LineOp:
             pass
 
 
+def plan_kernel(cls, kind, direction, bc3, dims, dd=1.0, alpha_f=0.0, lds_limit=160 * 1024):
+    """Name of the kernel that an operator on fields of dims runs, chosen on the host without a GPU."""
+    name = ctypes.create_string_buffer(128)
+    check(lib().mc3d_plan_kernel(cls, kind, direction, (ctypes.c_int * 3)(*bc3), (ctypes.c_int * 3)(*dims), dd,
+                                 alpha_f, lds_limit, name, len(name)))
+    return name.value.decode()
+
+
 def plan_tables(cls, kind, bc, n, dd=1.0, alpha_f=0.0, mm=0):
     """Host-built partition tables of an operator (diagnostic; no GPU needed)."""
     sizes = (ctypes.c_int * 11)()

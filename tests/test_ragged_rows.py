@@ -1,5 +1,5 @@
 """Ragged lines in 20- and 28-row chunks: lengths whose remainder over 16 or 32
-rows is too short for the interface blocks (65, 129, 193, ... points), and
+rows is too short for the interface blocks (65, 129, 193, 257, ... points), and
 y/z-lines of 257 to 320 points; and the chunk rows of evenly chunked y/z-lines."""
 import numpy as np
 import pytest
@@ -34,8 +34,72 @@ def test_plan_replay(monkeypatch, n, mm):
                         else (lambda f: P.filter_line(kind, bc, f, af)), n)
 
 
+@pytest.mark.parametrize("others", [(8, 9), (32, 24)])
+def test_every_length_has_a_kernel(others):
+    """Every operator is accepted on every length from 11 to 992 points, whatever
+    remainder 16- and 32-row chunks leave; 993 = 31 x 32 + 1 has no split that a
+    kernel takes, and a singular operator is refused as one at every length."""
+    from mpi_3dcompact_amd._lib import Mc3dError
+    from mpi_3dcompact_amd.ops import plan_kernel
+    short = (211, 226, 227, 241, 242, 243, 257, 258, 259, 289, 321, 322, 323, 353, 481, 609, 641, 737, 865, 961)
+    for n in [*range(11, 260, 3), *short, 992]:
+        for d in range(3):
+            dims = list(others)
+            dims.insert(d, n)
+            for cls, kind, af in OPS:
+                for bc in (P.PERIODIC, P.DIRICHLET):
+                    bc3 = [0, 0, 0]
+                    bc3[d] = bc
+                    assert plan_kernel(cls, kind, d, bc3, dims, 0.1, af).startswith("lineop_")
+    with pytest.raises(Mc3dError, match="cannot partition line"):
+        plan_kernel(1, P.COMPACT8, 1, (0, 0, 0), (32, 993, 24), 1.0, 0.49)
+    for n in (64, 257):
+        with pytest.raises(Mc3dError, match="zero pivot"):
+            plan_kernel(1, P.COMPACT8, 1, (0, 0, 0), (32, n, 24), 1.0, 1.0)
+
+
+def test_short_remainders_take_fast_kernels():
+    """512 lines or more of 32 k + 1 points (W = 2: + 2, + 3 too) in 20- or 28-row chunks."""
+    from mpi_3dcompact_amd.ops import plan_kernel
+    for n, mm in ((81, 28), (129, 20), (161, 28), (241, 28), (257, 20), (258, 20), (289, 20), (321, 28), (353, 28)):
+        for d in range(3):
+            dims = [32, 24]
+            dims.insert(d, n)
+            k = plan_kernel(0, P.PENTA10, d, (1, 1, 1), dims)
+            assert f", {mm}, false, ragged>" in k, (n, d, k)
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("n", [49, 65, 97, 129, 131, 193, 225, 305, 310])
+@pytest.mark.parametrize("n", [241, 257])
+@pytest.mark.parametrize("d", [0, 1, 2])
+def test_few_lines_of_short_remainders(n, d):
+    """Fewer than 512 lines, which take 32-row chunks, and the transformed-periodic
+    twin of the 20- and 28-row plans, which takes 32-row chunks as well."""
+    import torch
+    from mpi_3dcompact_amd.ops import LineOp
+    rng = np.random.default_rng(n + d)
+    for others in ([12, 11], [25, 24]):
+        dims = list(others)
+        dims.insert(d, n)
+        f = rng.normal(size=dims[::-1])
+        fin = torch.from_numpy(f).cuda()
+        out = torch.empty_like(fin)
+        for kind in (P.PADE6, P.PENTA10):
+            for bc in (P.PERIODIC, P.DIRICHLET):
+                op = LineOp.deriv(kind, d, bc, tuple(dims), 1.0 / n)
+                print(f"n={n} dir={d} kind={kind} bc={bc} {op.kernel()}", flush=True)
+                op.apply([fin], [out])
+                want = P.deriv_field(kind, d, bc, f, 1.0 / n)
+                assert np.max(np.abs(out.cpu().numpy() - want)) <= 1e-12 * np.max(np.abs(want)), (kind, bc)
+            op = LineOp.deriv(kind, d, P.PERIODIC, tuple(dims), 1.0 / n)
+            wraps = [rng.normal(size=others[0] * others[1]) for _ in range(6)]
+            op.apply_tpb(fin, out, [torch.from_numpy(w).cuda() for w in wraps])
+            want = P.deriv_field_tpb(kind, d, f, 1.0 / n, wraps)
+            assert np.max(np.abs(out.cpu().numpy() - want)) <= 1e-12 * np.max(np.abs(want)), kind
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [49, 65, 97, 129, 131, 193, 225, 241, 257, 289, 305, 310, 321])
 @pytest.mark.parametrize("d", [0, 1, 2])
 def test_lines_against_oracle(n, d):
     """Every banded operator on lines of n points among 24 x 24 others, both
