@@ -445,11 +445,11 @@ int mc3d_plan_tables(int cls, int kind, int bc, int n, double dd, double alphaF,
 
 /* Diagnostic (no counterpart in the reference): the name (mc3d_lineop_kernel)
  * of the kernel that plain applications of an operator in the MC3D_XPENCIL
- * layout run on a device whose workgroups may have lds_limit bytes of LDS,
- * chosen on the host without a GPU.  cls and kind as above; MC3D_EINVAL and
+ * layout run on a device of cus compute units whose workgroups may have
+ * lds_limit bytes of LDS, chosen on the host without a GPU.  cls and kind as above; MC3D_EINVAL and
  * MC3D_ENUMERIC where creating the operator gives them. */
 int mc3d_plan_kernel(int cls, int kind, int dir, const int bc3[3], const int dims[3], double dd, double alphaF,
-                     int lds_limit, char *name, int len);
+                     int lds_limit, int cus, char *name, int len);
 
 /* ---------------------------------------------------------------------------
  * Ensembles (no counterpart in the reference, which runs one box per job):

@@ -43,7 +43,7 @@ SIGNATURES = [
                                         ctypes.c_double, ctypes.c_double, ctypes.c_int, _I, _D, _D,
                                         _D, _D, _D, _D, _I, _I]),
     ("mc3d_plan_kernel", ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, _I, _I, ctypes.c_double,
-                                        ctypes.c_double, ctypes.c_int, ctypes.c_char_p, ctypes.c_int]),
+                                        ctypes.c_double, ctypes.c_int, ctypes.c_int, ctypes.c_char_p, ctypes.c_int]),
 ]
 
 _LIB = None

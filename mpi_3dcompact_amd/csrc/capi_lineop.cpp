@@ -80,50 +80,59 @@ int rotate(int layout, int dir, const int dims[3], const int bc3[3], int vd[3], 
 // an operator with an implicit part (W > 0)
 bool banded(int cls, int kind) { return cls == mc3d::kDeriv ? kind != MC3D_CD2 : kind != MC3D_COMMN5EXP; }
 
+// What the choice of a kernel depends on: LDS bytes that a workgroup may have, and
+// the CUs that a launch's workgroups (64 lines of one field each) spread over.
+struct Device {
+    int lds_limit, cus;
+};
+
 // Rows per chunk of evenly chunked y- and z-lines of banded operators, or 0 for
 // the plan's own choice (32 or 16 rows).  A workgroup is one wave per chunk, so
 // the chunk count sets how well workgroups pack into a CU's wave slots: 6, 8,
-// 12 or 16 chunks of 20, 24 or 28 rows (or four of 24) beat the 5 to 15 chunks
-// of 32 or 16 rows the same line splits into.  Four fields, y, 32 (or 16) rows
-// against these: 144 points Penta10 113 -> 93 us, 160 Compact10 104 -> 82, 192
-// Compact10 99 -> 84 and Penta10 101 -> 85, 224 CommN5Pade 105 -> 91, 240 Penta10
-// 124 -> 93, 288 Penta10 127 -> 96, 320 Pade6 101 -> 93, 384 Penta10 107 -> 104,
-// 448 105 -> 97, 96 91 -> 83.  (28 x 4 at 112 points was mixed; 128 and 256
-// points have no such split and keep 32.)  64 points: four chunks of 16 rows
-// instead of two of 32, which leave a 64^3 box 512 waves for 1024 SIMDs
-// (four fields: Pade6 7.7 -> 6.9 us, Penta10 8.6 -> 7.6, Compact10 10.0 -> 7.6).
-// Four chunks beyond 12288 lines no longer pay: the chip is full either way
-// (five fields: 64 points 0.93-0.98 of the time of 32 rows at 9216 lines, 1.05-1.2
-// at 16384; 96 points 0.89-0.92 and up to 1.13).  Compact10's wide window makes six
-// chunks of 24 rows slower than nine of 16 up to 24576 lines (1.04-1.06; 0.95 at
-// 36864 and more), where Penta10's take 0.79-0.87.
-int strided_rows(int cls, int kind, int n, long nlines) {
+// 12 or 16 chunks of 20, 24 or 28 rows beat the 5 to 15 chunks of 32 or 16 rows
+// that the same line splits into.  Four fields, y, 32 (or 16) rows against these:
+// 144 points Penta10 113 -> 93 us, 160 Compact10 104 -> 82, 192 Compact10 99 -> 84
+// and Penta10 101 -> 85, 224 CommN5Pade 105 -> 91, 240 Penta10 124 -> 93, 288
+// Penta10 127 -> 96, 320 Pade6 101 -> 93, 384 Penta10 107 -> 104, 448 105 -> 97.
+// (128 and 256 points have no such split and keep 32.)  The least gain: 144 points
+// up to 24576 lines with tridiagonal operators, five fields 0.84-1.05 of the time
+// of 16 rows, one field 0.99-1.08 (Penta10 0.70-1.03).
+// Lines that the plan splits into two or three chunks (64, 96 points) take four of
+// 16 or 24 rows while one field's workgroups fill at most three quarters of the
+// CUs: a 64^3 box is 512 waves in two chunks a line, for 1024 SIMDs (four fields:
+// Pade6 7.7 -> 6.9 us, Penta10 8.6 -> 7.6, Compact10 10.0 -> 7.6; 96 points 91 -> 83).
+// With more lines the chip is full either way (five fields, five operators: 64
+// points 0.86-1.01 of the time of 32 rows at 12288 lines, 1.05-1.25 at 20480; 96
+// points 0.89-0.96 at 9216, 0.91-1.12 at 12288, 0.94-1.10 at 24576).
+int strided_rows(int cls, int kind, int n, long nlines, const Device &hw) {
     if (!banded(cls, kind) || n % 16 != 0) return 0;
-    if (n <= 96 && nlines > 12288) return 0;
-    if (n / 32 == 2) return n % 32 ? 0 : 16;
-    if (n == 6 * 24 && cls == mc3d::kFilter && kind == MC3D_COMPACT10 && nlines <= 24576) return 0;
+    const int own = n % 32 == 0 && n > 32 ? n / 32 : n / 16;  // chunks of the plan's own choice
+    if (own < 4) return n >= 4 * 16 && 4 * ((nlines + 63) / 64) <= 3L * hw.cus ? n / 4 : 0;
     for (int mm : {24, 28, 20}) {
         const int P = n / mm;
-        if (n % mm == 0 && (P == 6 || P == 8 || P == 12 || P == 16 || (P == 4 && mm == 24))) return mm;
+        if (n % mm == 0 && (P == 6 || P == 8 || P == 12 || P == 16)) return mm;
     }
     return 0;
 }
 
 // Rows per chunk with which lineop_contig_groups takes x-lines of n points of a
-// banded operator (half bandwidth W), Dirichlet or ragged, or 0: four or eight
-// chunks, whose waves spread evenly over a CU's SIMDs (the fewest rows that give
-// at most so many; 144 points: eight chunks of 20 rows 3.6-4.0 TB/s, six of 24
+// banded operator (half bandwidth W), Dirichlet or ragged, or 0: at most four or
+// eight chunks, whose waves spread evenly over a CU's SIMDs (the fewest rows that
+// give so few; 144 points: eight chunks of 20 rows 3.6-4.0 TB/s, six of 24
 // 2.9-3.4).  113 to 128 points are eight 16-row chunks, which the whole tile serves
-// as well.  The second workgroup of a CU is the gain, so a launch has to have one:
-// with up to 16384 lines a field is 256 workgroups, and one field of 160 to 256
-// points takes 1.0-1.5 times the whole tile's time (four fields 1.0-1.4 up to 4096
-// lines, 0.7-0.9 from 6144 on); at 17408 lines 0.72-0.90.  Whole tiles of up to 112
-// points fit a CU three at a time and win up to 32768 lines of one field (1.06-1.3;
-// 0.75-1.02 at 49152).  Unevenly chunked lines below 160 points gain at any count
-// (129-158 points 0.86-1.02 at 4096 lines, 0.59-1.02 beyond).
-int grouped_rows(int n, int W, long nlines) {
+// as well.  The second workgroup of a CU is the gain, so a launch has to have one.
+// An operator is planned before the number of fields of a launch is known, so one
+// field decides: with a workgroup a CU (16384 lines on 256 CUs) one field of 160 to
+// 256 points takes 1.0-1.5 times the whole tile's time, at 17408 lines 0.72-0.90
+// (four fields at once would gain from 6144 lines on: 0.7-0.9, 1.0-1.4 up to 4096).
+// Whole tiles of up to 112 points fit a CU three at a time and win up to two
+// workgroups a CU (one field 1.06-1.3 at 32768 lines; 0.75-1.02 at 49152, three a
+// CU).  Unevenly chunked lines below 160 points gain from a quarter of a workgroup
+// a CU on (129-158 points 0.86-1.02 at 4096 lines, 0.59-1.02 beyond).
+int grouped_rows(int n, int W, long nlines, const Device &hw) {
     if (n < 96 || n > 256 || (n > 112 && n <= 128)) return 0;
-    if (nlines < (n <= 112 ? 49152 : n < 160 && n % 16 ? 4096 : 16385)) return 0;
+    const long full = 64L * hw.cus;  // lines of one workgroup a CU
+    if (nlines < (n <= 112 ? 3 * full : n < 160 && n % 16 ? full / 4 : full + 1)) return 0;
     const int chunks = n <= 112 ? 4 : 8;
     for (int mm : {20, 24, 28, 32}) {
         const int P = (n + mm - 1) / mm, rem = n - (P - 1) * mm;
@@ -148,12 +157,11 @@ int check_request(int cls, int dir, int bc, const int dims[3], double dd, int nb
     return MC3D_OK;
 }
 
-// Plan, kernel and launch shape of an operator (all but its device tables), for a
-// device whose workgroups may have lds_limit bytes of LDS.
+// Plan, kernel and launch shape of an operator (all but its device tables).
 int choose(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[3], double dd, double alphaF,
-           int nbatch, const mc3d::LineTune &tune, int lds_limit, mc3d_lineop *op) {
+           int nbatch, const mc3d::LineTune &tune, const Device &hw, mc3d_lineop *op) {
     const long npts = (long)dims[0] * dims[1] * dims[2] * nbatch;
-    op->lds_limit = lds_limit;
+    op->lds_limit = hw.lds_limit;
     std::string err;
     bool groups = false;  // plan for lineop_contig_groups
     auto plan_with = [&](int mm) -> int {
@@ -190,9 +198,9 @@ int choose(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
         const bool offsets_ok = npts * 8 < 4294967296L;
         d.groups = groups ? 1 : 0;
         d.phases = 1;
-        if (!groups) d.phases = mc3d::lineop_fast_phases(d, (size_t)lds_limit);
+        if (!groups) d.phases = mc3d::lineop_fast_phases(d, (size_t)hw.lds_limit);
         op->fast = (p.uniform || p.cshort >= 0) && rows_ok && offsets_ok &&
-                   mc3d::lineop_fast_supported(d, (size_t)lds_limit);
+                   mc3d::lineop_fast_supported(d, (size_t)hw.lds_limit);
         if (tune.family == 2) op->fast = false;
         return MC3D_OK;
     };
@@ -226,7 +234,7 @@ int choose(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
     };
     std::vector<int> cand{tune.mm};
     if (!tune.mm) {
-        const int first = dir == 0 ? (dims[0] % 16 == 0 ? 16 : 0) : strided_rows(cls, kind, dims[dir], nlines);
+        const int first = dir == 0 ? (dims[0] % 16 == 0 ? 16 : 0) : strided_rows(cls, kind, dims[dir], nlines, hw);
         cand = first ? std::vector<int>{first, 0, 16} : std::vector<int>{0, 16};
     }
     bool found = false, tried16 = false;
@@ -268,7 +276,7 @@ int choose(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
         op->fast = false;
     }
     if (auto_rows && dir == 0 && (bc == MC3D_DIRICHLET || op->plan.cshort >= 0)) {
-        const int mm = grouped_rows(dims[0], op->plan.W, nlines);
+        const int mm = grouped_rows(dims[0], op->plan.W, nlines, hw);
         if (mm > 0) {
             const mc3d::Plan whole = op->plan;
             const mc3d::OpDev dev = op->dev;
@@ -313,12 +321,14 @@ int create(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
     *out = nullptr;
     int rc = check_request(cls, dir, bc, dims, dd, nbatch, tune);
     if (rc) return rc;
-    int dev = 0, lds_limit = 65536;
+    int dev = 0;
+    Device hw{65536, 256};
     if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&lds_limit, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
+        hipDeviceGetAttribute(&hw.lds_limit, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
+        hipDeviceGetAttribute(&hw.cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return mc3d::fail(MC3D_EHIP, "cannot query the device");
     auto *op = new mc3d_lineop();
-    rc = choose(cls, kind, dir, bc, bc3, dims, dd, alphaF, nbatch, tune, lds_limit, op);
+    rc = choose(cls, kind, dir, bc, bc3, dims, dd, alphaF, nbatch, tune, hw, op);
     if (rc) {
         delete op;
         return rc;
@@ -479,14 +489,14 @@ int mc3d_plan_tables(int cls, int kind, int bc, int n, double dd, double alphaF,
 }
 
 int mc3d_plan_kernel(int cls, int kind, int dir, const int bc3[3], const int dims[3], double dd, double alphaF,
-                     int lds_limit, char *name, int len) {
+                     int lds_limit, int cus, char *name, int len) {
     if (!bc3 || !name || len < 1) return mc3d::fail(MC3D_EINVAL, "null argument");
     if (dir < 0 || dir > 2) return mc3d::fail(MC3D_EINVAL, "dir must be 0, 1 or 2");
     const mc3d::LineTune t{};
     int rc = check_request(cls, dir, bc3[dir], dims, dd, 1, t);
     if (rc) return rc;
     mc3d_lineop op;
-    rc = choose(cls, kind, dir, bc3[dir], cls == mc3d::kFilter ? bc3 : nullptr, dims, dd, alphaF, 1, t, lds_limit, &op);
+    rc = choose(cls, kind, dir, bc3[dir], cls == mc3d::kFilter ? bc3 : nullptr, dims, dd, alphaF, 1, t, Device{lds_limit, cus}, &op);
     if (rc) return rc;
     if ((int)op.kname.size() >= len) return mc3d::fail(MC3D_EINVAL, "name buffer too small");
     std::memcpy(name, op.kname.c_str(), op.kname.size() + 1);

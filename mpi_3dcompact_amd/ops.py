@@ -104,11 +104,11 @@ class LineOp:
             pass
 
 
-def plan_kernel(cls, kind, direction, bc3, dims, dd=1.0, alpha_f=0.0, lds_limit=160 * 1024):
+def plan_kernel(cls, kind, direction, bc3, dims, dd=1.0, alpha_f=0.0, lds_limit=160 * 1024, cus=256):
     """Name of the kernel that an operator on fields of dims runs, chosen on the host without a GPU."""
     name = ctypes.create_string_buffer(128)
     check(lib().mc3d_plan_kernel(cls, kind, direction, (ctypes.c_int * 3)(*bc3), (ctypes.c_int * 3)(*dims), dd,
-                                 alpha_f, lds_limit, name, len(name)))
+                                 alpha_f, lds_limit, cus, name, len(name)))
     return name.value.decode()
 
 

@@ -69,6 +69,18 @@ def test_short_remainders_take_fast_kernels():
             assert f", {mm}, false, ragged>" in k, (n, d, k)
 
 
+@pytest.mark.parametrize("cus", [32, 256, 304])
+def test_rules_follow_the_device(cus):
+    """Four chunks of y/z-lines, and x-lines in groups, by workgroups (64 lines) a CU."""
+    from mpi_3dcompact_amd.ops import plan_kernel
+    def rows(d, dims):
+        return plan_kernel(0, P.PENTA10, d, (1, 1, 1), dims, cus=cus)
+    for n, four in ((64, 16), (96, 24)):
+        assert f", {four}, " in rows(2, (48 * cus, 1, n)) and ", 32, " in rows(2, (48 * cus + 1, 1, n))
+    for n, lines in ((112, 3 * 64 * cus), (150, 16 * cus), (160, 64 * cus + 1), (256, 64 * cus + 1)):
+        assert "_groups<" in rows(0, (n, lines, 1)) and "_groups<" not in rows(0, (n, lines - 1, 1)), n
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [241, 257])
 @pytest.mark.parametrize("d", [0, 1, 2])
@@ -151,8 +163,7 @@ def test_even_rows(n, mm, d):
             bc3 = [0, 0, 0]
             bc3[d] = bc
             op = LineOp.deriv(kind, d, bc, dims, dd) if cls == 0 else LineOp.filter(kind, af, d, bc3, dims)
-            rows = 16 if n == 144 and (cls, kind) == (1, P.COMPACT10) else mm
-            assert f", {rows}, " in op.kernel() and op.kernel().startswith("lineop_strided<"), op.kernel()
+            assert f", {mm}, " in op.kernel() and op.kernel().startswith("lineop_strided<"), op.kernel()
             want = P.deriv_field(kind, d, bc, f, dd) if cls == 0 else P.filter_field(kind, af, d, bc3, f)
             out = torch.empty_like(fin)
             op.apply([fin], [out])
