@@ -332,6 +332,7 @@ int mc3d_solver_timing(mc3d_solver *s, int enable) {
     return guarded([&] {
         s->cs->timer.reset();
         s->cs->timer.enable(enable != 0);
+        if (enable) s->cs->countMetricFields();
     });
 }
 

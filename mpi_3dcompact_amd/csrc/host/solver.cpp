@@ -458,10 +458,12 @@ CurvilinearCSolver::CurvilinearCSolver(const Options &o, hipStream_t s, int memb
     hip_check(hipMalloc(&p, sizeof(StepScalars) * members), "scalar allocation");
     extra_.push_back(p);
     sc = static_cast<StepScalars *>(p);
-    hip_check(hipMalloc(&p, sizeof(int)), "metric flag");
+    const std::vector<int> unset((size_t)members + 1, 1);
+    hip_check(hipMalloc(&p, sizeof(int) * unset.size()), "metric flags");
     extra_.push_back(p);
     msh.varies = planes_vary_ = static_cast<int *>(p);
-    checkMetricPlanes();
+    hip_check(hipMemcpy(p, unset.data(), sizeof(int) * unset.size(), hipMemcpyHostToDevice), "metric flags");
+    metrics_set_.assign((size_t)members, 0);
     const std::vector<StepScalars> s0((size_t)members, StepScalars{opt.dt, opt.CFL, opt.time, 0.0});
     hip_check(hipMemcpy(sc, s0.data(), sizeof(StepScalars) * members, hipMemcpyHostToDevice), "scalar init");
     if (members > 1) {
@@ -591,10 +593,26 @@ double *CurvilinearCSolver::alloc_field() {
 // The flag lives on the device and is set again with every change of the
 // metrics, so captured steps read the current one.  A metric field whose device
 // address the caller holds may change at any time: its planes count as different.
-void CurvilinearCSolver::checkMetricPlanes() {
-    hip_check(metrics_exposed_ ? launch_set_int(planes_vary_, 1, st) : launch_metric_planes(msh, planes_vary_, N, st),
-              "metric planes");
-    int varies = 1;  // a copy for the byte counts of the launch timings
+// Stacked members keep a flag each, so that setting one member reads that member
+// alone (the first one, whose first plane all are compared with, also those set
+// before it).
+void CurvilinearCSolver::checkMetricPlanes(int b) {
+    if (metrics_exposed_) {
+        hip_check(launch_set_int(planes_vary_, 1, st), "metric planes");
+    } else if (dom.members == 1) {
+        hip_check(launch_metric_planes(msh, 0, N, planes_vary_, st), "metric planes");
+    } else {
+        metrics_set_[(size_t)b] = 1;
+        for (int m = 0; m < dom.members; ++m)
+            if (m == b || (b == 0 && metrics_set_[(size_t)m]))
+                hip_check(launch_metric_planes(msh, (long)m * dom.gN, dom.gN, planes_vary_ + 1 + m, st), "metric planes");
+        hip_check(launch_any_int(planes_vary_ + 1, dom.members, planes_vary_, st), "metric planes");
+    }
+    if (timer.enabled()) countMetricFields();
+}
+
+void CurvilinearCSolver::countMetricFields() {
+    int varies = 1;
     hip_check(hipMemcpyAsync(&varies, planes_vary_, sizeof(int), hipMemcpyDeviceToHost, st), "metric planes");
     hip_check(hipStreamSynchronize(st), "metric planes");
     metric_fields_ = varies ? 10.0 : 0.0;
@@ -664,7 +682,7 @@ void CurvilinearCSolver::setMemberMetrics(int b, const double *const m[10]) {
     for (int k = 0; k < 10; ++k)
         hip_check(hipMemcpyAsync(Jm[k] + off, m[k], sizeof(double) * dom.gN, hipMemcpyHostToDevice, st),
                   "metric upload");
-    checkMetricPlanes();
+    checkMetricPlanes(b);
     hip_check(hipStreamSynchronize(st), "metric upload");
 }
 

@@ -321,8 +321,9 @@ class CurvilinearCSolver {
     Metrics msh{};
     double *Jm[10] = {};
     bool div_apart_ = false;         // eta and zeta divergences in tmp[0..4], tmp[5..9]
-    int *planes_vary_ = nullptr;     // Metrics::varies
-    double metric_fields_ = 10.0;    // metric fields k_flux and k_vreman stream (0: the first plane)
+    int *planes_vary_ = nullptr;     // Metrics::varies, then (stacked members) each member's own flag
+    std::vector<char> metrics_set_;  // stacked members whose metrics were given
+    double metric_fields_ = 10.0;    // metric fields k_flux and k_vreman stream (0: the first plane), when timed
     bool metrics_exposed_ = false;   // a metric field's address was handed out
     Cons r1{}, rk_{}, k2{}, r2{};
     Prim pr{};
@@ -344,8 +345,10 @@ class CurvilinearCSolver {
     void set_metrics_host(const double *const m[10]);
     // field_by_name for callers that keep the address
     double *expose_field(const std::string &name);
-    // sets *planes_vary_ from the metric fields
-    void checkMetricPlanes();
+    // sets *planes_vary_ from the metric fields, of which member b's have changed
+    void checkMetricPlanes(int b = 0);
+    // reads it back for the byte counts of timed launches
+    void countMetricFields();
     // metrics from mesh coordinates (device x, y, z), src/AbstractSingleBlockMesh.cpp:23-1309
     void solveForJacobians(const double *x, const double *y, const double *z);
     void set_mesh_host(const double *x, const double *y, const double *z);

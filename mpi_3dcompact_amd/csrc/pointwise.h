@@ -121,10 +121,12 @@ hipError_t launch_cfl_finish(const double *partial, int nblocks, StepScalars *sc
 // the same maxima into out[2 b] = cfl / maxspeed, out[2 b + 1] = maxspeed of each member
 hipError_t launch_cfl_out(const double *partial, int nblocks, int nmember, double cfl, double *out,
                           hipStream_t st);
-// *varies = 1 if any of the ten metric fields (n points) differs in any bit
-// between z-planes of `plane` points, else 0
-hipError_t launch_metric_planes(const Metrics &m, int *varies, long n, hipStream_t st);
+// *varies = 1 if any of the ten metric fields differs in any bit, in a z-plane
+// among the n points from `first` on, from the first plane of the field, else 0
+hipError_t launch_metric_planes(const Metrics &m, long first, long n, int *varies, hipStream_t st);
 hipError_t launch_set_int(int *p, int v, hipStream_t st);
+// *any = whether one of n flags is set
+hipError_t launch_any_int(const int *flags, int n, int *any, hipStream_t st);
 hipError_t launch_flux(const FluxArgs &a, Gas g, long n, hipStream_t st);
 hipError_t launch_rhs_rk(const RkArgs &a, long n, hipStream_t st);
 hipError_t launch_vreman(const double *const dU[3], const double *const dV[3],

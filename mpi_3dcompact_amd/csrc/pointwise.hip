@@ -441,19 +441,27 @@ __global__ __launch_bounds__(kBlock) void k_vreman(VremanArgs a, unsigned plane)
 struct MetricList {
     const double *f[10];
 };
-__global__ __launch_bounds__(kBlock) void k_metric_planes(MetricList m, unsigned plane, long n, int *varies) {
+__global__ __launch_bounds__(kBlock) void k_metric_planes(MetricList m, unsigned plane, long first, unsigned n,
+                                                          int *varies) {
     if (*(volatile int *)varies) return;
     bool differ = false;
-    for (long ip = (long)blockIdx.x * kBlock + threadIdx.x; ip < n; ip += (long)gridDim.x * kBlock) {
-        const long jp = ip % plane;
+    for (unsigned i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+        const unsigned jp = i % plane;
 #pragma unroll
         for (int k = 0; k < 10; ++k)
-            differ |= __double_as_longlong(m.f[k][ip]) != __double_as_longlong(m.f[k][jp]);
+            differ |= __double_as_longlong(m.f[k][first + i]) != __double_as_longlong(m.f[k][jp]);
     }
     if (differ) atomicOr(varies, 1);
 }
 
 __global__ void k_set_int(int *p, int v) { *p = v; }
+
+__global__ __launch_bounds__(kBlock) void k_any_int(const int *flags, int n, int *any) {
+    int f = 0;
+    for (int i = threadIdx.x; i < n; i += kBlock) f |= flags[i];
+    f = __syncthreads_or(f);
+    if (threadIdx.x == 0) *any = f != 0;
+}
 
 __global__ void k_fill(double *p, double v, long n) {
     const long ip = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -648,14 +656,19 @@ hipError_t launch_cfl_out(const double *partial, int nblocks, int nmember, doubl
     return hipGetLastError();
 }
 
-hipError_t launch_metric_planes(const Metrics &m, int *varies, long n, hipStream_t st) {
-    if (m.plane == 0 || n % m.plane) return launch_set_int(varies, 1, st);
+hipError_t launch_metric_planes(const Metrics &m, long first, long n, int *varies, hipStream_t st) {
+    if (m.plane == 0 || n % m.plane || n > 0x7fffffffL) return launch_set_int(varies, 1, st);
     const MetricList l{{m.J, m.J11, m.J12, m.J13, m.J21, m.J22, m.J23, m.J31, m.J32, m.J33}};
     const hipError_t e = launch_set_int(varies, 0, st);
     if (e != hipSuccess) return e;
     const long b = (n + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(k_metric_planes, dim3((unsigned)(b < 16384 ? b : 16384)), dim3(kBlock), 0, st, l, m.plane, n,
-                       varies);
+    hipLaunchKernelGGL(k_metric_planes, dim3((unsigned)(b < 16384 ? b : 16384)), dim3(kBlock), 0, st, l, m.plane, first,
+                       (unsigned)n, varies);
+    return hipGetLastError();
+}
+
+hipError_t launch_any_int(const int *flags, int n, int *any, hipStream_t st) {
+    hipLaunchKernelGGL(k_any_int, dim3(1), dim3(kBlock), 0, st, flags, n, any);
     return hipGetLastError();
 }
 
