@@ -147,26 +147,17 @@ __global__ __launch_bounds__(kBlock) void k_cfl_out(const double *partial, int n
 }
 
 // ---------------------------------------------------------------------------
-// k_flux and k_vreman run over z-planes (blockIdx.y).  Where the mesh repeats
-// its first z-plane (Metrics::varies) the metric terms are read from that
-// plane, which the caches hold; else every point streams its own.  Ten of
-// k_flux's 48 fields and of k_vreman's 21 then leave the HBM traffic (256^3 box:
-// 5.37 -> 4.61 and 2.27 -> 1.41 ms of a step, 5.5 and 5.2 TB/s of what is left).
+// Where the mesh repeats its first z-plane (Metrics::varies) k_flux and k_vreman
+// read the metric terms from that plane, which the caches hold; else every point
+// streams its own.  Ten of k_flux's 48 fields and of k_vreman's 21 then leave the
+// HBM traffic (256^3 box: 5.37 -> 4.61 and 2.27 -> 1.41 ms of a step, 5.5 and
+// 5.2 TB/s of what is left).  The point of the plane is a remainder of the flat
+// index: a grid row per plane rounds every plane up to whole workgroups
+// (k_flux of 17 x 17 x 2048 points: 41.6 us streaming, 54.9 with grid rows, 36.3 so;
+// 250 x 13 x 512: 114, 116, 94; 256^3 the same either way).
 // A thread walking several planes with the terms in registers spilled 325
 // scalar registers (the 48 field addresses stay live around the loop).
 // ---------------------------------------------------------------------------
-struct PlaneGrid {
-    dim3 grid;
-    unsigned plane;
-};
-inline PlaneGrid plane_grid(const Metrics &m, long n) {
-    const bool whole = !m.plane || n % m.plane || n / m.plane > 65535;  // no planes to share
-    PlaneGrid c;
-    c.plane = whole ? (unsigned)n : m.plane;
-    c.grid = dim3((c.plane + kBlock - 1) / kBlock, (unsigned)(n / c.plane));
-    return c;
-}
-
 struct MetricPoint {
     double J, J11, J12, J13, J21, J22, J23, J31, J32, J33;
 };
@@ -183,6 +174,10 @@ __device__ __forceinline__ MetricPoint load_metrics(const Metrics &m, long i) {
         q.J31 = ldm<STREAM>(m.J31, i); q.J32 = ldm<STREAM>(m.J32, i); q.J33 = ldm<STREAM>(m.J33, i);
     }
     return q;
+}
+__device__ __forceinline__ MetricPoint metrics_at(const Metrics &m, long ip) {
+    if (!m.varies || *m.varies) return load_metrics<true>(m, ip);
+    return load_metrics<false>(m, (unsigned)ip % m.plane);  // (fields of fewer than 2^31 points)
 }
 
 // Stress, heat flux and contravariant fluxes / J, src/CurvilinearCSolver_Core.cpp:548-561,615-752
@@ -263,12 +258,10 @@ __device__ __forceinline__ void flux_point(const FluxArgs &a, const Gas &g, cons
     stnt(a.pre[4], ip, iJ * (F1 - G1)); stnt(a.pre[9], ip, iJ * (F2 - G2)); stnt(a.pre[14], ip, iJ * (F3 - G3));
 }
 
-__global__ __launch_bounds__(kBlock) void k_flux(FluxArgs a, Gas g, unsigned plane) {
-    const unsigned jp = blockIdx.x * kBlock + threadIdx.x;
-    if (jp >= plane) return;
-    const long ip = (long)blockIdx.y * plane + jp;
-    const MetricPoint mp = !a.m.varies || *a.m.varies ? load_metrics<true>(a.m, ip) : load_metrics<false>(a.m, jp);
-    flux_point(a, g, mp, ip);
+__global__ __launch_bounds__(kBlock) void k_flux(FluxArgs a, Gas g, long n) {
+    const long ip = (long)blockIdx.x * kBlock + threadIdx.x;
+    if (ip >= n) return;
+    flux_point(a, g, metrics_at(a.m, ip), ip);
 }
 
 // one conserved variable: k2 and the register update of stage op; returns the
@@ -428,11 +421,10 @@ __device__ __forceinline__ void vreman_point(const VremanArgs &a, const MetricPo
     stnt(a.mu_sgs, ip, ms < cap ? ms : cap);
 }
 
-__global__ __launch_bounds__(kBlock) void k_vreman(VremanArgs a, unsigned plane) {
-    const unsigned jp = blockIdx.x * kBlock + threadIdx.x;
-    if (jp >= plane) return;
-    const long ip = (long)blockIdx.y * plane + jp;
-    const MetricPoint mp = !a.m.varies || *a.m.varies ? load_metrics<true>(a.m, ip) : load_metrics<false>(a.m, jp);
+__global__ __launch_bounds__(kBlock) void k_vreman(VremanArgs a, long n) {
+    const long ip = (long)blockIdx.x * kBlock + threadIdx.x;
+    if (ip >= n) return;
+    const MetricPoint mp = metrics_at(a.m, ip);
     vreman_point(a, mp, filter_width2(a.dx, a.dy, a.dz, mp.J), ip);
 }
 
@@ -678,8 +670,7 @@ hipError_t launch_set_int(int *p, int v, hipStream_t st) {
 }
 
 hipError_t launch_flux(const FluxArgs &a, Gas g, long n, hipStream_t st) {
-    const PlaneGrid c = plane_grid(a.m, n);
-    hipLaunchKernelGGL(k_flux, c.grid, dim3(kBlock), 0, st, a, g, c.plane);
+    hipLaunchKernelGGL(k_flux, grid_for(n), dim3(kBlock), 0, st, a, g, n);
     return hipGetLastError();
 }
 
@@ -692,8 +683,7 @@ hipError_t launch_vreman(const double *const dU[3], const double *const dV[3],
                          const double *const dW[3], Metrics m, const double *rho, double *mu_sgs,
                          double dx, double dy, double dz, long n, hipStream_t st) {
     const VremanArgs a{{dU[0], dU[1], dU[2]}, {dV[0], dV[1], dV[2]}, {dW[0], dW[1], dW[2]}, m, rho, mu_sgs, dx, dy, dz};
-    const PlaneGrid c = plane_grid(m, n);
-    hipLaunchKernelGGL(k_vreman, c.grid, dim3(kBlock), 0, st, a, c.plane);
+    hipLaunchKernelGGL(k_vreman, grid_for(n), dim3(kBlock), 0, st, a, n);
     return hipGetLastError();
 }
 

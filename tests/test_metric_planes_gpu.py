@@ -46,7 +46,7 @@ def extruded(dims):
                             (nz, ny, nx)).copy() for b in base]
 
 
-@pytest.mark.parametrize("dims", [(32, 32, 32), (13, 12, 36), (64, 20, 16)])
+@pytest.mark.parametrize("dims", [(32, 32, 32), (13, 12, 36), (64, 20, 16), (17, 17, 40)])
 def test_repeated_planes_give_the_same_bits(dims):
     m = extruded(dims)
     a, b = run(dims, m, False), run(dims, m, True)
