@@ -50,8 +50,8 @@ struct AdamArgs {
 hipError_t launch_mlp_reduce_adam(const float *partial, const float *lossp, int nblocks, long n_total, float *loss,
                                   float *params, float *m, float *v, AdamArgs a, hipStream_t st);
 hipError_t launch_mlp_adam(float *params, float *m, float *v, const float *grad, AdamArgs a, hipStream_t st);
-// Y[n][2] = network(X[n][7]) on standardised values (the register-resident
-// inference path the solver uses)
+// Y[n][2] = network(X[n][7]) on standardised values (the products of the solver's
+// kernels, the network staged in LDS)
 hipError_t launch_mlp_infer(const float *params, const float *X, float *Y, long n, hipStream_t st);
 
 // The seven raw features of every point (FP32 values stored as FP64 fields),

@@ -1,5 +1,5 @@
-// Learned SGS closure kernels: training (gradient, reduction, Adam), the
-// register-resident inference path, the fused per-point closure of the solver
+// Learned SGS closure kernels: training (gradient, reduction, Adam), inference
+// with the network staged in LDS, the fused per-point closure of the solver
 // step, its DSM fallback merge, and training-pair sampling from a DSM state.
 //
 // Matrix products use v_mfma_f32_16x16x32_bf16 (gfx950).  Operand layout of
@@ -8,7 +8,8 @@
 //   B[k][j]: lane holds j = l % 16, k = 8 g + e
 //   D[i][j]: lane holds j = l % 16, i = 4 g + r (r = 0..3)
 // Compiled with -ffp-contract=off: the FP32 and FP64 scalar arithmetic is
-// rounded once per operation, as the checker restates it.
+// rounded once per operation, except for the fused step in the GELU's exponent;
+// biases enter a product as its accumulator.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -22,12 +23,6 @@ namespace {
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ unsigned short f2bf(float f) {
-    unsigned u = __float_as_uint(f);
-    u += 0x7fffu + ((u >> 16) & 1u);  // round to nearest even (finite inputs)
-    return (unsigned short)(u >> 16);
-}
 
 __device__ __forceinline__ f32x4 mfma(const s16x8 &a, const s16x8 &b, const f32x4 &c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b),
@@ -61,8 +56,7 @@ __device__ __forceinline__ float gelu_grad(float z, float s) {
 
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63); }
 
-// FP32 -> BF16 by the hardware conversion (round to nearest even, as f2bf for
-// finite values)
+// FP32 -> BF16 by the hardware conversion (round to nearest even)
 __device__ __forceinline__ short bf16_bits(float v) { return __builtin_bit_cast(short, (__bf16)v); }
 
 __device__ __forceinline__ int kappa(int b, int g, int e) { return 16 * (2 * b + (e >> 2)) + 4 * g + (e & 3); }
@@ -102,11 +96,12 @@ struct TrainLds {
     float red[4][3 * kMlpHid + kMlpOut + 1]; // per-wave sums: three bias gradients, db4, squares
 };
 
-// the operands of wave w (row and column tile w of every matrix) for the lane
-// (i = lane % 16, g = lane / 16), converted from the FP32 parameters; the
-// four waves' shares are equal and straight-line, so every load is in flight
-// before the first conversion
-__device__ __forceinline__ void stage_train(const float *__restrict__ P, TrainLds &s, int w, int l) {
+// the operands of wave w (row tile w of every matrix; TRAIN: column tiles too, for
+// the backward products) for the lane (i = lane % 16, g = lane / 16), converted
+// from the FP32 parameters; the four waves' shares are equal and straight-line, so
+// every load is in flight before the first conversion
+template <bool TRAIN>
+__device__ __forceinline__ void stage_operands(const float *__restrict__ P, s16x8 (*ops)[64], int w, int l) {
     const int i = l & 15, g = l >> 4;
     float r1[8], c4[2], c3[2][8], c2[2][8];
     f32x4 r[3][2][2];
@@ -122,23 +117,25 @@ __device__ __forceinline__ void stage_train(const float *__restrict__ P, TrainLd
             r[1][b][hi] = *reinterpret_cast<const f32x4 *>(P + kMlpOffW3 + (16 * w + i) * kMlpHid + col);
             r[2][b][hi] = *reinterpret_cast<const f32x4 *>(P + kMlpOffW4 + (i < kMlpOut ? i : 0) * kMlpHid + col);
         }
+    if constexpr (TRAIN) {
 #pragma unroll
-    for (int o = 0; o < kMlpOut; ++o) c4[o] = P[kMlpOffW4 + o * kMlpHid + 16 * w + i];
+        for (int o = 0; o < kMlpOut; ++o) c4[o] = P[kMlpOffW4 + o * kMlpHid + 16 * w + i];
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+        for (int b = 0; b < 2; ++b)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            c3[b][e] = P[kMlpOffW3 + kappa(b, g, e) * kMlpHid + 16 * w + i];
-            c2[b][e] = P[kMlpOffW2 + kappa(b, g, e) * kMlpHid + 16 * w + i];
-        }
+            for (int e = 0; e < 8; ++e) {
+                c3[b][e] = P[kMlpOffW3 + kappa(b, g, e) * kMlpHid + 16 * w + i];
+                c2[b][e] = P[kMlpOffW2 + kappa(b, g, e) * kMlpHid + 16 * w + i];
+            }
+    }
     s16x8 o1, o4;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         o1[e] = g == 0 ? bf16_bits(r1[e]) : (short)0;
-        o4[e] = g == 0 && e < kMlpOut ? bf16_bits(c4[e < kMlpOut ? e : 0]) : (short)0;
+        if constexpr (TRAIN) o4[e] = g == 0 && e < kMlpOut ? bf16_bits(c4[e < kMlpOut ? e : 0]) : (short)0;
     }
-    s.w[w][l] = o1;
-    s.w[22 + w][l] = o4;
+    ops[w][l] = o1;
+    if constexpr (TRAIN) ops[22 + w][l] = o4;
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
         s16x8 o2, o3, o2t, o3t, o4r;
@@ -147,14 +144,18 @@ __device__ __forceinline__ void stage_train(const float *__restrict__ P, TrainLd
             o2[e] = bf16_bits(r[0][b][e >> 2][e & 3]);
             o3[e] = bf16_bits(r[1][b][e >> 2][e & 3]);
             o4r[e] = i < kMlpOut ? bf16_bits(r[2][b][e >> 2][e & 3]) : (short)0;
-            o3t[e] = bf16_bits(c3[b][e]);
-            o2t[e] = bf16_bits(c2[b][e]);
+            if constexpr (TRAIN) {
+                o3t[e] = bf16_bits(c3[b][e]);
+                o2t[e] = bf16_bits(c2[b][e]);
+            }
         }
-        s.w[4 + 2 * w + b][l] = o2;
-        s.w[12 + 2 * w + b][l] = o3;
-        if (w == 0) s.w[20 + b][l] = o4r;
-        s.w[26 + 2 * w + b][l] = o3t;
-        s.w[34 + 2 * w + b][l] = o2t;
+        ops[4 + 2 * w + b][l] = o2;
+        ops[12 + 2 * w + b][l] = o3;
+        if (w == 0) ops[20 + b][l] = o4r;
+        if constexpr (TRAIN) {
+            ops[26 + 2 * w + b][l] = o3t;
+            ops[34 + 2 * w + b][l] = o2t;
+        }
     }
 }
 
@@ -240,7 +241,7 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ P, c
     for (int e = 0; e < 8; ++e)
         x[e] = (g == 0 && ok && e < kMlpIn) ? bf16_bits(X[src * kMlpIn + (e < kMlpIn ? e : 0)]) : (short)0;
     const float t0 = ok ? Tg[src * kMlpOut] : 0.0f, t1 = ok ? Tg[src * kMlpOut + 1] : 0.0f;
-    stage_train(P, s, w, l);
+    stage_operands<true>(P, s.w, w, l);
     if (tid < 3 * kMlpHid)
         s.b[tid / kMlpHid][tid % kMlpHid] =
             P[(tid < kMlpHid ? kMlpOffB1 : tid < 2 * kMlpHid ? kMlpOffB2 : kMlpOffB3) + tid % kMlpHid];
@@ -504,34 +505,22 @@ __device__ __forceinline__ void features(const double A[3][3], double vol_J, flo
 // The network stays in LDS and a wave's weight operands are loaded into
 // registers only around the products of each 64-point group: the FP64 feature
 // phase and the network phase then do not hold their registers at the same
-// time (4 waves per SIMD instead of 1).  Per-lane
+// time (3 waves per SIMD instead of 1).  Per-lane
 // operands are stored [operand][lane] as 16-byte entries (w1 t = 0..3, w2 t,b,
 // w3 t,b, w4 b), biases by neuron.
 // ---------------------------------------------------------------------------
-constexpr int kWOps = 4 + 8 + 8 + 2;
 struct InferLds {
-    s16x8 w[kWOps][64];
+    s16x8 w[kFwdOps][64];
     float b[3][kMlpHid];
     float b4[4];  // zero beyond the two outputs
 };
 
-// the operands, written entry by entry by the whole workgroup
+// the operands and biases, by a workgroup of four waves.  (Entry by entry, 44
+// loads and conversions a thread one after another, k_mlp_infer of up to 60000
+// samples, at most one group a wave, took 16.4-18.0 us; 9.2 so, 300000 samples
+// 39.5 -> 24.9, k_learned_sgs of 160^3 points 332 -> 307.)
 __device__ void stage_infer(const float *__restrict__ P, InferLds &s) {
-    for (int idx = threadIdx.x; idx < kWOps * 64 * 8; idx += blockDim.x) {
-        const int e = idx & 7, l = (idx >> 3) & 63, op = idx >> 9;
-        const int i = l & 15, g = l >> 4;
-        float v;
-        if (op < 4) {
-            const int k = 8 * g + e;
-            v = k < kMlpIn ? P[kMlpOffW1 + (16 * op + i) * kMlpIn + k] : 0.0f;
-        } else if (op < 20) {
-            const int q = op < 12 ? op - 4 : op - 12, t = q >> 1, b = q & 1;
-            v = P[(op < 12 ? kMlpOffW2 : kMlpOffW3) + (16 * t + i) * kMlpHid + kappa(b, g, e)];
-        } else {
-            v = i < kMlpOut ? P[kMlpOffW4 + i * kMlpHid + kappa(op - 20, g, e)] : 0.0f;
-        }
-        reinterpret_cast<short *>(&s.w[op][l])[e] = (short)f2bf(v);
-    }
+    stage_operands<false>(P, s.w, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane_id());
     for (int k = threadIdx.x; k < 3 * kMlpHid; k += blockDim.x) {
         const int layer = k / kMlpHid, j = k % kMlpHid;
         s.b[layer][j] = P[(layer == 0 ? kMlpOffB1 : layer == 1 ? kMlpOffB2 : kMlpOffB3) + j];
