@@ -475,7 +475,8 @@ int mc3d_ensemble_set_initial(mc3d_ensemble *e, int member, const double *rho0, 
                               const double *V0, const double *W0, const double *p0);
 /* Measure and select, per box size and direction, the launch shape of the
  * derivative and filter operators (rows per chunk, kernel family, lines per
- * workgroup).  cache_path (NULL: none) is a text file of earlier results, read
+ * workgroup; small boxes' derivatives keep the default where the launch that
+ * their three directions then share is faster).  cache_path (NULL: none) is a text file of earlier results, read
  * first and written back with the new ones.  Synchronous. */
 int mc3d_ensemble_tune(mc3d_ensemble *e, const char *cache_path);
 int mc3d_ensemble_step(mc3d_ensemble *e, int nsteps);
@@ -488,7 +489,9 @@ int mc3d_ensemble_scalars(mc3d_ensemble *e, int member, double *time, double *dt
 int mc3d_ensemble_stream(mc3d_ensemble *e, void **stream);
 int mc3d_ensemble_sync(mc3d_ensemble *e);
 /* JSON: buckets (box size, members, kernels of the derivative and filter
- * operators per direction, tuning results), graphs captured, graph launches.
+ * operators per direction, whether the x, y and z derivatives of the 4 gradient
+ * fields and of the 5 fluxes share a launch, tuning results), graphs captured,
+ * graph launches.
  * MC3D_EINVAL if buf is too small (the required size goes to *needed). */
 int mc3d_ensemble_info(mc3d_ensemble *e, char *buf, int buflen, int *needed);
 void mc3d_ensemble_destroy(mc3d_ensemble *e);

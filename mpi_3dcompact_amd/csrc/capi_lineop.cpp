@@ -535,31 +535,45 @@ int lineop_launch_accumulate(const mc3d_lineop *op, const double *const *in, dou
     return apply(op, in, out, nfields, mode, nullptr, accumulate, stream);
 }
 
-int lineop_launch_together(const mc3d_lineop *const ops[3], const double *const *const in[3],
-                           double *const *const out[3], int n, bool &done, void *stream) {
-    done = false;
-    if (n < 1 || 3 * n > kMaxFields) return MC3D_OK;
-    OpSet o{};
-    LaunchArgs a{};
+namespace {
+// the operators as one launch's, or false where they do not make one
+bool op_set(const mc3d_lineop *const ops[3], OpSet &o) {
     const mc3d_lineop *f = ops[0];
     for (int d = 0; d < 3; ++d) {
         const mc3d_lineop *op = ops[d];
         if (!op->fast || op->cls != kDeriv || op->dir != d || op->nbatch != f->nbatch ||
             std::memcmp(op->dims, f->dims, sizeof(op->dims)))
-            return MC3D_OK;
+            return false;
         o.op[d] = op->dev;
         o.nlines[d] = (int)((long)op->dims[0] * op->dims[1] * op->dims[2] * (d == 2 ? 1 : op->nbatch) / op->dims[d]);
+    }
+    return true;
+}
+}  // namespace
+
+bool lineop_shares_launch(const mc3d_lineop *const ops[3], int n) {
+    OpSet o{};
+    return n >= 1 && 3 * n <= kMaxFields && op_set(ops, o) &&
+           lineop_together_supported(o, n, ops[0]->nbatch, (size_t)ops[0]->lds_limit);
+}
+
+int lineop_launch_together(const mc3d_lineop *const ops[3], const double *const *const in[3],
+                           double *const *const out[3], int n, bool &done, void *stream) {
+    done = lineop_shares_launch(ops, n);
+    if (!done) return MC3D_OK;
+    OpSet o{};
+    op_set(ops, o);
+    LaunchArgs a{};
+    for (int d = 0; d < 3; ++d)
         for (int k = 0; k < n; ++k) {
             a.in[d * n + k] = in[d][k];
             a.out[d * n + k] = out[d][k];
         }
-    }
+    const mc3d_lineop *f = ops[0];
     a.Nx = f->dims[0]; a.Ny = f->dims[1]; a.Nz = f->dims[2];
     a.nbatch = f->nbatch;
-    if (!lineop_together_supported(o, n, f->nbatch, (size_t)f->lds_limit)) return MC3D_OK;
     const hipError_t e = lineop_launch_together(o, a, n, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(MC3D_EHIP, std::string("line operator launch: ") + hipGetErrorString(e));
-    done = true;
     return MC3D_OK;
 }
 }  // namespace mc3d

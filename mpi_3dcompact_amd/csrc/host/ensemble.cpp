@@ -41,6 +41,72 @@ std::string json_escape(const std::string &s) {
     return o;
 }
 
+// milliseconds of `once` on st, after a warm-up
+template <typename F>
+double time_launches(F &&once, hipEvent_t e0, hipEvent_t e1, hipStream_t st) {
+    once();
+    const int reps = 3;
+    hip_check(hipEventRecord(e0, st), "tuning");
+    for (int r = 0; r < reps; ++r) once();
+    hip_check(hipEventRecord(e1, st), "tuning");
+    hip_check(hipEventSynchronize(e1), "tuning");
+    float ms = 0.f;
+    hip_check(hipEventElapsedTime(&ms, e0, e1), "tuning");
+    return (double)ms / reps;
+}
+
+// a bucket's three default derivative operators, which share a launch in small boxes
+class SharedDerivs {
+  public:
+    SharedDerivs(CurvilinearCSolver &cs, const int dims[3], const Options::FDType ft[3], const double dd[3], int nm,
+                 hipStream_t st)
+        : cs_(cs), st_(st) {
+        const int bc3[3] = {MC3D_PERIODIC, MC3D_PERIODIC, MC3D_PERIODIC};
+        for (int d = 0; d < 3; ++d)
+            if (lineop_create(kDeriv, fd_scheme(ft[d]), d, bc3, dims, dd[d], 0.0, nm, LineTune{}, &op_[d]) != MC3D_OK)
+                return;
+        for (int k = 0; k < 2; ++k) share_[k] = lineop_shares_launch(op_, 4 + k);
+    }
+    ~SharedDerivs() {
+        for (mc3d_lineop *op : op_) mc3d_lineop_destroy(op);
+    }
+    SharedDerivs(const SharedDerivs &) = delete;
+    SharedDerivs &operator=(const SharedDerivs &) = delete;
+    bool possible() const { return share_[0] || share_[1]; }
+    // the derivatives of a stage: 4 gradient fields, then 5 fluxes, whose parts come apart
+    // where they share a launch (the stage update adds them: ten fields more read
+    // there, which the accumulating launches read otherwise; at 5 TB/s)
+    double time(hipEvent_t e0, hipEvent_t e1) {
+        const double ms = time_launches([&] { stage(4); stage(5); }, e0, e1, st_);
+        return ms + (share_[1] ? 10.0 * 8.0 * (double)cs_.N / 5e9 : 0.0);
+    }
+
+  private:
+    CurvilinearCSolver &cs_;
+    hipStream_t st_;
+    mc3d_lineop *op_[3] = {};
+    bool share_[2] = {};
+
+    void stage(int n) {
+        const double *in4[4] = {cs_.pr.U, cs_.pr.V, cs_.pr.W, cs_.pr.T};
+        const double *in[3][5];
+        double *out[3][5];
+        for (int d = 0; d < 3; ++d)
+            for (int k = 0; k < n; ++k) {
+                double *grad[4] = {cs_.dU[d], cs_.dV[d], cs_.dW[d], cs_.dT[d]};
+                in[d][k] = n == 4 ? in4[k] : cs_.pre[5 * d + k];
+                out[d][k] = n == 4 ? grad[k] : d == 0 || !share_[1] ? cs_.div[k] : cs_.tmp[5 * (d - 1) + k];
+            }
+        const double *const *ins[3] = {in[0], in[1], in[2]};
+        double *const *outs[3] = {out[0], out[1], out[2]};
+        bool done = false;
+        int rc = lineop_launch_together(op_, ins, outs, n, done, st_);
+        for (int d = 0; d < 3 && !done && rc == MC3D_OK; ++d)
+            rc = lineop_launch_accumulate(op_[d], in[d], out[d], n, n == 5 && d > 0, st_);
+        if (rc != MC3D_OK) throw Error(rc, "tuning launch failed");
+    }
+};
+
 }  // namespace
 
 Ensemble::Ensemble(const Options &opt, int members, const int *dims, const double *mu) : opt_(opt) {
@@ -216,6 +282,10 @@ void Ensemble::dropGraphs() {
 // derivative of 4 fields (velocity and temperature gradients) plus a
 // derivative of 5 fields added into the divergence; a filter of the 5
 // conserved fields.  Outputs go to work fields the step overwrites anyway.
+// Small boxes' default derivative operators share one launch for x, y and z
+// (lineop_together), which needs one shape in all three directions: there the
+// shared launch is timed against the three directions' best shapes together, and
+// all three keep the default where it wins.
 void Ensemble::tune(const std::string &cache_path) {
     dropGraphs();
     std::map<std::string, std::string> cache;
@@ -250,20 +320,28 @@ void Ensemble::tuneBucket(Bucket &b, std::map<std::string, std::string> &cache) 
     hip_check(hipEventCreate(&e1), "event creation");
     LineTune dsh[3], fsh[3];
     b.tuned.clear();
+    SharedDerivs shared(cs, b.dims, ft, dd, nm, b.st);
+    auto key_of = [&](int cls, int d) {
+        char key[256];
+        if (cls == 0)
+            std::snprintf(key, sizeof(key), "deriv %s periodic %dx%dx%d members %d dir %d%s", fd_name(ft[d]),
+                          b.dims[0], b.dims[1], b.dims[2], nm, d, shared.possible() ? " or shared" : "");
+        else
+            std::snprintf(key, sizeof(key), "filter %s alpha %.6g periodic %dx%dx%d members %d dir %d",
+                          fkind == MC3D_COMPACT8 ? "COMPACT8" : "COMPACT10", opt_.alphaF, b.dims[0], b.dims[1],
+                          b.dims[2], nm, d);
+        return std::string(key);
+    };
+    // (the three directions of a choice that includes the shared launch belong together)
+    bool derivs_cached = true;
+    for (int d = 0; d < 3; ++d) derivs_cached = derivs_cached && cache.count(key_of(0, d));
     for (int cls = 0; cls < 2; ++cls)
         for (int d = 0; d < 3; ++d) {
-            char key[256];
-            if (cls == 0)
-                std::snprintf(key, sizeof(key), "deriv %s periodic %dx%dx%d members %d dir %d", fd_name(ft[d]),
-                              b.dims[0], b.dims[1], b.dims[2], nm, d);
-            else
-                std::snprintf(key, sizeof(key), "filter %s alpha %.6g periodic %dx%dx%d members %d dir %d",
-                              fkind == MC3D_COMPACT8 ? "COMPACT8" : "COMPACT10", opt_.alphaF, b.dims[0],
-                              b.dims[1], b.dims[2], nm, d);
+            const std::string key = key_of(cls, d);
             TunedShape best;
             best.key = key;
             auto hit = cache.find(key);
-            if (hit != cache.end() && parse_shape(hit->second, best)) {
+            if (hit != cache.end() && (cls == 1 || derivs_cached || !shared.possible()) && parse_shape(hit->second, best)) {
                 best.cached = true;
             } else {
                 best.ms = -1.0;
@@ -287,15 +365,7 @@ void Ensemble::tuneBucket(Bucket &b, std::map<std::string, std::string> &cache) 
                                 throw Error(MC3D_EHIP, "tuning launch failed");
                         }
                     };
-                    once();  // warm-up
-                    const int reps = 3;
-                    hip_check(hipEventRecord(e0, b.st), "tuning");
-                    for (int r = 0; r < reps; ++r) once();
-                    hip_check(hipEventRecord(e1, b.st), "tuning");
-                    hip_check(hipEventSynchronize(e1), "tuning");
-                    float ms = 0.f;
-                    hip_check(hipEventElapsedTime(&ms, e0, e1), "tuning");
-                    return (double)ms / reps;
+                    return time_launches(once, e0, e1, b.st);
                 };
                 // candidates: the untuned default first (the plan's own
                 // chunking, which for line lengths such as 40, 72 or 200 is an
@@ -333,11 +403,20 @@ void Ensemble::tuneBucket(Bucket &b, std::map<std::string, std::string> &cache) 
                         best.shape = t;
                     }
                 }
-                if (best.candidates == 0) throw Error(MC3D_EINVAL, std::string("no launch shape for ") + key);
+                if (best.candidates == 0) throw Error(MC3D_EINVAL, "no launch shape for " + key);
                 cache[key] = format_shape(best);
             }
             (cls == 0 ? dsh : fsh)[d] = best.shape;
             b.tuned.push_back(best);
+            if (cls == 0 && d == 2 && shared.possible() && !derivs_cached) {
+                const double ms = shared.time(e0, e1);
+                if (ms < b.tuned[0].ms + b.tuned[1].ms + b.tuned[2].ms)
+                    for (int k = 0; k < 3; ++k) {
+                        dsh[k] = b.tuned[k].shape = LineTune{};
+                        b.tuned[k].ms = ms / 3.0;
+                        cache[key_of(0, k)] = format_shape(b.tuned[k]);
+                    }
+            }
         }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
@@ -364,6 +443,10 @@ std::string Ensemble::info() const {
         for (int d = 0; d < 3; ++d)
             o << (d ? ", " : "") << "\""
               << json_escape(lineop_kernel_name(static_cast<const LineFilter *>(fv[d])->op())) << "\"";
+        const mc3d_lineop *ops[3];
+        cs.derivOps(ops);
+        o << "], \"shared\": [" << (lineop_shares_launch(ops, 4) ? "true" : "false") << ", "
+          << (lineop_shares_launch(ops, 5) ? "true" : "false");
         o << "], \"tuned\": [";
         for (size_t k = 0; k < b.tuned.size(); ++k) {
             const TunedShape &t = b.tuned[k];

@@ -1104,10 +1104,14 @@ void CurvilinearCSolver::gradientsAndSGS() {
     }
 }
 
+void CurvilinearCSolver::derivOps(const mc3d_lineop *ops[3]) const {
+    const AbstractDerivatives *dv[3] = {derivX.get(), derivY.get(), derivZ.get()};
+    for (int d = 0; d < 3; ++d) ops[d] = static_cast<const LineDerivative *>(dv[d])->op();
+}
+
 bool CurvilinearCSolver::derivsTogether(int n, const double *const *const in[3], double *const *const out[3]) {
-    AbstractDerivatives *dv[3] = {derivX.get(), derivY.get(), derivZ.get()};
     const mc3d_lineop *ops[3];
-    for (int d = 0; d < 3; ++d) ops[d] = static_cast<LineDerivative *>(dv[d])->op();
+    derivOps(ops);
     bool done = false;
     const int t = timer.begin("lineop_together", 3.0 * n * 16.0 * (double)N);
     mc3d_check(lineop_launch_together(ops, in, out, n, done, st), "derivatives");

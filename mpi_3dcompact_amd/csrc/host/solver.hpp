@@ -380,6 +380,7 @@ class CurvilinearCSolver {
     void preSubStep();            // preStepDerivatives
     // derivatives of n fields along x, y, z (in[d] -> out[d]) in one launch; false,
     // and nothing done, where that does not pay
+    void derivOps(const mc3d_lineop *ops[3]) const;  // the operators along x, y, z
     bool derivsTogether(int n, const double *const *const in[3], double *const *const out[3]);
     void gradientsAndSGS();       //   its derivative and SGS part
     void flux();                  //   its flux and divergence part

@@ -16,6 +16,7 @@ int lineop_launch_accumulate(const mc3d_lineop *op, const double *const *in, dou
 // otherwise
 int lineop_launch_together(const mc3d_lineop *const ops[3], const double *const *const in[3],
                            double *const *const out[3], int n, bool &done, void *stream);
+bool lineop_shares_launch(const mc3d_lineop *const ops[3], int n);
 
 // Launch shape of a line operator: rows per chunk (16 or 32; 0 chooses),
 // kernel family (0 chooses: the fast kernels when they take the operator;

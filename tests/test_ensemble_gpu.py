@@ -192,3 +192,23 @@ def test_ensemble_refuses_what_it_does_not_batch(gpu):
     e = Ensemble(hit.options_text(32), [(32,) * 3, (16,) * 3])
     with pytest.raises(Mc3dError):
         e.step(1)  # nothing set
+
+
+def test_tuning_keeps_the_launch_that_small_boxes_share(gpu, tmp_path):
+    """Boxes whose default derivatives go along x, y and z in one launch keep it
+    unless the three directions' best shapes are faster together: two 56^3 members
+    lost it to a 16-row x operator that was faster by itself.  The choice is cached."""
+    members = [dict(N=n, Mt=0.3, mu=1e-3, seed=k) for k, n in enumerate((32, 56, 56, 96))]
+    cache = tmp_path / "shapes.txt"
+    # an entry of a cache written before the shared launch was compared does not decide
+    cache.write_text("deriv PADE6 periodic 56x56x56 members 2 dir 0 = 16 1 0 0.000001 13\n")
+    plain = build(members, **C3).info()["buckets"]
+    assert [b["shared"] for b in plain] == [[True, True], [True, True], [False, False]]
+    first = build(members, tune=True, tune_cache=cache, **C3).info()["buckets"]
+    again = build(members, tune=True, tune_cache=cache, **C3).info()["buckets"]
+    for b, c, p in zip(first, again, plain):
+        _say(b["dims"], b["shared"], b["deriv"], [t["ms"] for t in b["tuned"][:3]])
+        assert b["shared"] == p["shared"] and c["shared"] == b["shared"]
+        assert c["deriv"] == b["deriv"] and all(t["cached"] for t in c["tuned"])
+        if p["shared"][0]:
+            assert b["deriv"] == p["deriv"]
