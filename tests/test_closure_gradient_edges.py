@@ -31,19 +31,28 @@ def test_gradient_at_partial_tiles(n):
 
 
 def test_training_batch_equals_gradient_and_adam():
-    """One epoch of one whole batch visits every sample once: the same update as
-    gradient() and adam_step() up to the order of the sums (weights move by at
-    most lr = 1e-3; a gradient entry off by 1e-4 of itself moves its weight by
-    less than 1e-3 of that unless the entry is rounding noise)."""
+    """Three epochs of one whole batch each visit every sample once: the same
+    updates as gradient() and adam_step() up to the order of the FP32 sums.  Two
+    orders' gradients differ by at most 2e-8 here (700 samples), so a step of an
+    entry of gradient |g| differs by lr 2e-8 / |g| and by the rounding of a weight
+    below 1 (6e-8): 8e-8 from |g| = 1e-3 on, 2e-6 from 1e-5 on, three steps of that.
+    A partial sum left out turns the sign, and so the whole step of lr, of many
+    such entries."""
     import torch
     from mpi_3dcompact_amd.closure import Closure
     r = np.random.default_rng(3)
     X = torch.from_numpy(r.standard_normal((700, 7)).astype(np.float32)).cuda()
     T = torch.from_numpy(r.standard_normal((700, 2)).astype(np.float32)).cuda()
     a, b = Closure(4), Closure(4)
-    (loss,) = a.train(X, T, epochs=1, batch=700, lr=1e-3, seed=9)
-    g, want = b.gradient(X, T)
-    b.adam_step(g, lr=1e-3)
-    assert abs(loss - want) <= 1e-6 * want
+    losses = a.train(X, T, epochs=3, batch=700, lr=1e-3, seed=9)
+    least = np.full(b.params().size, np.inf)
+    for loss in losses:
+        g, want = b.gradient(X, T)
+        b.adam_step(g, lr=1e-3)
+        assert abs(loss - want) <= 1e-6 * want
+        least = np.minimum(least, np.abs(g.cpu().numpy()))
+    assert np.abs(b.params()).max() < 1.0
     d = np.abs(a.params() - b.params())
-    assert np.quantile(d, 0.99) <= 1e-6 and d.max() <= 2e-3
+    big, most = least >= 1e-3, least >= 1e-5
+    assert big.mean() >= 0.3 and most.mean() >= 0.97
+    assert d[big].max() <= 2.5e-7 and d[most].max() <= 6e-6

@@ -16,10 +16,18 @@ def gpu():
         pytest.skip("no GPU")
 
 
-def run(dims, metrics, own, again=None, steps=2):
+def streamed(s, n):
+    """Metric fields that k_flux reads point by point: 10, or 0 where it reads one plane."""
+    s.timing(True)
+    s.step(1)
+    (k,) = [r for r in s.timing_report() if r["kernel"] == "k_flux"]
+    return round(k["bytes"] / (8 * n * k["count"])) - 38  # 22 other fields and mu_sgs read, 15 written
+
+
+def run(dims, metrics, own, again=None, steps=2, fields=None):
     """Conserved and k2 fields after some steps; own: every point streams its own
     metric terms (a metric field's address was handed out); again: metrics set
-    after the first step."""
+    after the first step; fields: how many metric fields must stream then."""
     from mpi_3dcompact_amd.solver import Solver
     shape = dims[::-1]
     s = Solver(hit.options_text(dims[0], fd="PADE6", filt="COMPACT8", rk="KENRK4", les="VREMAN", les_avg="NONE",
@@ -34,7 +42,10 @@ def run(dims, metrics, own, again=None, steps=2):
     if again is not None:
         s.set_metrics(again)
     s.step(steps - 1)
-    return {n: s.field(n) for n in ("rho", "rhoU", "rhoV", "rhoW", "rhoE", "rhok2", "rhoUk2", "rhoEk2", "sos", "mu_sgs")}
+    out = {n: s.field(n) for n in ("rho", "rhoU", "rhoV", "rhoW", "rhoE", "rhok2", "rhoUk2", "rhoEk2", "sos", "mu_sgs")}
+    if fields is not None:
+        assert streamed(s, dims[0] * dims[1] * dims[2]) == fields
+    return out
 
 
 def extruded(dims):
@@ -49,22 +60,24 @@ def extruded(dims):
 @pytest.mark.parametrize("dims", [(32, 32, 32), (13, 12, 36), (64, 20, 16), (17, 17, 40)])
 def test_repeated_planes_give_the_same_bits(dims):
     m = extruded(dims)
-    a, b = run(dims, m, False), run(dims, m, True)
+    a, b = run(dims, m, False, fields=0), run(dims, m, True, fields=10)
     for k in a:
         assert np.all(np.isfinite(a[k])) and np.array_equal(a[k], b[k]), k
 
 
 @pytest.mark.parametrize("field", [0, 2, 9])
 def test_one_point_of_the_last_plane(field):
-    """A single value off by one bit in the last plane makes the planes differ."""
+    """A single value off by one bit in the last plane makes the planes differ, and
+    one off by a hundredth shows in the results."""
     dims = (32, 16, 16)
     m = extruded(dims)
-    m[field][-1, -1, -1] = np.nextafter(m[field][-1, -1, -1], 10.0) * (1.0 + 0.01)
-    a, b = run(dims, m, False), run(dims, m, True)
+    m[field][-1, -1, -1] = np.nextafter(m[field][-1, -1, -1], 10.0)
+    a, b = run(dims, m, False, fields=10), run(dims, m, True)
+    m[field][-1, -1, -1] *= 1.01
+    c, d = run(dims, m, False, fields=10), run(dims, m, True)
     for k in a:
-        assert np.array_equal(a[k], b[k]), k
-    c = run(dims, extruded(dims), False)
-    assert not np.array_equal(a["rhoE"], c["rhoE"])
+        assert np.array_equal(a[k], b[k]) and np.array_equal(c[k], d[k]), k
+    assert not np.array_equal(c["rhoE"], run(dims, extruded(dims), False)["rhoE"])
 
 
 def test_metrics_set_again():
@@ -73,7 +86,7 @@ def test_metrics_set_again():
     m, v = extruded(dims), extruded(dims)
     v[5][3:] *= 1.02
     for first, second in ((m, v), (v, m)):
-        a, b = run(dims, first, False, again=second), run(dims, first, True, again=second)
+        a, b = run(dims, first, False, again=second, fields=10 if second is v else 0), run(dims, first, True, again=second)
         for k in a:
             assert np.array_equal(a[k], b[k]), k
 

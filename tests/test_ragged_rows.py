@@ -111,7 +111,7 @@ def test_few_lines_of_short_remainders(n, d):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n", [49, 65, 97, 129, 131, 193, 225, 241, 257, 289, 305, 310, 321])
+@pytest.mark.parametrize("n", [49, 65, 81, 97, 129, 131, 161, 193, 225, 241, 257, 289, 305, 310, 321])
 @pytest.mark.parametrize("d", [0, 1, 2])
 def test_lines_against_oracle(n, d):
     """Every banded operator on lines of n points among 24 x 24 others, both
@@ -191,7 +191,8 @@ def test_grouped_x_lines(n):
             dd = 1.0 / n if bc == P.PERIODIC else 1.0 / (n - 1)
             op = LineOp.deriv(kind, 0, bc, dims, dd) if cls == 0 else LineOp.filter(kind, af, 0, bc3, dims)
             print(f"n={n} cls={cls} kind={kind} bc3={bc3} {op.kernel()}", flush=True)
-            if bc == P.DIRICHLET:
+            # periodic lines that split evenly (by 16 rows, 200 by 20) keep the 16-line tiles
+            if bc == P.DIRICHLET or (n % 16 and n != 200):
                 assert op.kernel().startswith("lineop_contig_groups<"), op.kernel()
             sub = np.ascontiguousarray(f[ends])
             want = P.deriv_field(kind, 0, bc, sub, dd) if cls == 0 else P.filter_field(kind, af, 0, list(bc3), sub)
@@ -202,6 +203,32 @@ def test_grouped_x_lines(n):
                 op.apply([same], [same])
                 assert torch.equal(same, out)
             assert np.max(np.abs(out.cpu().numpy()[ends] - want)) <= 1e-12 * np.max(np.abs(want)), (cls, kind, bc3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [97, 131, 160, 193, 230, 256])
+@pytest.mark.parametrize("bc", [P.PERIODIC, P.DIRICHLET])
+def test_grouped_x_lines_accumulate(n, bc):
+    """out += derivative, which the library's internal entry asks for (no public one
+    does along x), to the bit the sum of the plain result and what was there."""
+    import ctypes
+    import torch
+    from mpi_3dcompact_amd import lib
+    from mpi_3dcompact_amd.ops import LineOp
+    add = getattr(lib(), "_ZN4mc3d24lineop_launch_accumulateEPK11mc3d_lineopPKPKdPKPdiiPv")
+    add.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
+    dims = (n, 33, 528 if n > 112 else 1504)
+    for kind in (P.PADE6, P.PENTA10):
+        op = LineOp.deriv(kind, 0, bc, dims, 1.0 / n)
+        if bc == P.DIRICHLET or n % 16:
+            assert op.kernel().startswith("lineop_contig_groups<"), op.kernel()
+        f = torch.rand(dims[::-1], dtype=torch.float64, device="cuda")
+        plain, out = torch.empty_like(f), torch.rand_like(f)
+        want = out.clone()
+        op.apply([f], [plain])
+        pi, po = (ctypes.c_void_p * 1)(f.data_ptr()), (ctypes.c_void_p * 1)(out.data_ptr())
+        assert add(op._h, pi, po, 1, 1, torch.cuda.current_stream().cuda_stream) == 0
+        assert torch.equal(out, want + plain), (n, kind)
 
 
 @pytest.mark.gpu

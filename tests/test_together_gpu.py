@@ -18,7 +18,7 @@ def gpu():
         pytest.skip("no GPU")
 
 
-@pytest.mark.parametrize("n,members,les", [(36, 11, None), (48, 6, "VREMAN"), (56, 4, None), (60, 4, None), (64, 3, "VREMAN")])
+@pytest.mark.parametrize("n,members,les", [(36, 11, None), (48, 6, "VREMAN"), (56, 7, None), (60, 4, None), (64, 3, "VREMAN")])
 @pytest.mark.parametrize("fd", ["PADE6", "PENTA10"])
 def test_shared_launch_equals_separate_launches(n, members, les, fd):
     from mpi_3dcompact_amd.ensemble import Ensemble
@@ -29,6 +29,7 @@ def test_shared_launch_equals_separate_launches(n, members, les, fd):
     mu = [1e-3 / (1 + m) for m in range(members)]
     start = [hit.hit_initial_condition(n, k0=4.0, Mt=0.3, seed=m) for m in range(members)]
     e = Ensemble(hit.options_text(n, **case), [(n,) * 3] * members, mu)
+    assert e.info()["buckets"][0]["shared"] == [False, False]
     for m in range(members):
         e.set_metrics(m, hit.identity_metrics(n))
         e.set_initial(m, start[m])
