@@ -122,9 +122,18 @@ void Closure::train(const float *X, const float *T, long n, int epochs, int batc
     // An epoch's visiting order depends on the seed alone: the next epoch's is
     // drawn while the GPU works on this one (262144 pairs, batches of 8192: an
     // order takes 0.45 ms on the host, its batches 0.58 ms on the GPU; four
-    // epochs 4.15 -> 3.30 ms)
+    // epochs 4.15 -> 3.3-3.5 ms)
     std::vector<int> order[2];
     std::vector<float> bl((size_t)nbatches);
+    // the stream's copies from and into these are done before they go, also when
+    // drawing an order runs out of memory or a launch fails
+    struct Wait {
+        hipStream_t s;
+        bool pending;
+        ~Wait() {
+            if (pending) (void)hipStreamSynchronize(s);
+        }
+    } wait{st, false};
     std::mt19937_64 rng(seed);
     auto draw_order = [&](std::vector<int> &o) {
         o.resize((size_t)n);
@@ -136,6 +145,7 @@ void Closure::train(const float *X, const float *T, long n, int epochs, int batc
     };
     draw_order(order[0]);
     for (int e = 0; e < epochs; ++e) {
+        wait.pending = true;
         hip_check(hipMemcpyAsync(idx_, order[e & 1].data(), sizeof(int) * (size_t)n, hipMemcpyHostToDevice, st),
                   "closure sample order");
         for (long b = 0; b < nbatches; ++b) {
@@ -150,6 +160,7 @@ void Closure::train(const float *X, const float *T, long n, int epochs, int batc
         hip_check(hipMemcpyAsync(bl.data(), loss_, sizeof(float) * (size_t)nbatches, hipMemcpyDeviceToHost, st),
                   "closure losses");
         hip_check(hipStreamSynchronize(st), "closure epoch");
+        wait.pending = false;
         double acc = 0.0;
         for (long b = 0; b < nbatches; ++b) acc += (double)bl[(size_t)b] * (double)std::min<long>(batch, n - b * batch);
         if (losses) losses[e] = acc / (double)n;
