@@ -163,8 +163,8 @@ def host_cpu():
 
 
 def cpu_baseline(n_cpu, steps=3, n_one=128):
-    """Oracle step rate on the host (test infrastructure, used only as the
-    checker/baseline): 1 warm-up and `steps` timed steps at n_cpu^3 on the
+    """Oracle step rate on the host (test infrastructure, used only as a
+    baseline): 1 warm-up and `steps` timed steps at n_cpu^3 on the
     threads OpenMP gives the oracle, then one step at n_one^3 on one thread."""
     from mpi_3dcompact_amd import hit
     from oracle import pyoracle as P

@@ -326,6 +326,11 @@ int mc3d_solver_hit_stats(mc3d_solver *s, double stats[11]);
  * with 17 significant digits and followed by a space, as the driver's
  * ofstream with precision(17) writes them.  NULL or "" switches it off. */
 int mc3d_solver_set_turbdata(mc3d_solver *s, const char *path, int every);
+/* Device address of a field (names as mc3d_solver_get_field).  Who holds the
+ * address of a metric field (J, J11 .. J33) may write it at any time, so from
+ * then on the solver reads the metrics of every point, also after a later
+ * mc3d_solver_set_metrics, where it otherwise reads one z-plane of a mesh whose
+ * planes repeat. */
 int mc3d_solver_field_device(mc3d_solver *s, const char *name, double **dev_ptr);
 /* Running statistics ([STATS] VELOCITYSTATS / THERMOSTATS, src/Stats.hpp):
  * their accumulated weights (the time they cover); the fields are read with

@@ -3,7 +3,7 @@
  *
  * TEST INFRASTRUCTURE ONLY.  This library is a plain-C++ restatement of the
  * reference algorithm (emathew1/MPI_3DCompact), used by tests/, by
- * __graft_entry__.smoke() and by bench.py's cpu_baseline leg as the checker.
+ * __graft_entry__.smoke() and by bench.py's cpu_baseline leg.
  * It is never linked into, loaded by, or called from the product library
  * (mpi_3dcompact_amd/), and the product path has no CPU fallback.
  *

@@ -21,7 +21,7 @@ Numerics the GPU kernels follow and this file restates:
 - every matrix product takes BF16 operands (round to nearest even) and
   accumulates in FP32 (here: exactly, in FP64, then rounded once);
 - biases, GELU, the loss and Adam in FP32.
-This file is NumPy only and is the checker; nothing in the product imports it.
+This file is NumPy only and is the oracle; nothing in the product imports it.
 """
 import numpy as np
 

@@ -1,5 +1,5 @@
 """Test infrastructure, not product code: a CPU restatement of the image
-outputs (the checker of the library's PNG writer), and a PNG decoder.
+outputs (the oracle of the library's PNG writer), and a PNG decoder.
 
 colormap(): src/PngWriter.hpp:270-313 (RAINBOW, BWR) and the GREYSCALE case
 of src/CurvilinearCSolver_Core.cpp:1729-1733; the colour scaling of

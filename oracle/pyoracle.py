@@ -1,7 +1,7 @@
 """ctypes view of the CPU oracle (oracle/liboracle.so).
 
 TEST INFRASTRUCTURE ONLY: imported by tests/, by __graft_entry__.smoke() and by
-bench.py's cpu_baseline leg, as the checker.  The product package never imports
+bench.py's cpu_baseline leg.  The product package never imports
 this module.
 """
 import ctypes

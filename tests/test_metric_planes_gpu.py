@@ -86,7 +86,7 @@ def test_metrics_set_again():
     m, v = extruded(dims), extruded(dims)
     v[5][3:] *= 1.02
     for first, second in ((m, v), (v, m)):
-        a, b = run(dims, first, False, again=second, fields=10 if second is v else 0), run(dims, first, True, again=second)
+        a, b = run(dims, first, False, again=second, fields=10 if second is v else 0), run(dims, first, True, again=second, fields=10)
         for k in a:
             assert np.array_equal(a[k], b[k]), k
 
