@@ -243,8 +243,8 @@ int choose(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
         found = fast_with(mm);
         tried16 = tried16 || op->plan.MM == 16;
     }
-    // Banded ragged lines of 512 lines or more, in 20-row chunks (28 where those
-    // leave the short chunk fewer than 2W rows) and one short chunk:
+    // Banded ragged lines of 512 lines or more, in at most 16 20-row chunks (28
+    // where those leave the short chunk fewer than 2W rows) and one short chunk:
     //  - lines whose remainder over 16 (32) rows is too short for its interface
     //    blocks (65, 129, 193, 257 points, say), which only the LDS-tiled kernel
     //    takes otherwise: 129-point Penta10 y in a 160 x 129 x 144 box, four
@@ -254,9 +254,8 @@ int choose(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
     //    Penta10 z 231 -> 200 us against 32-row chunks (4.0 -> 4.6 TB/s), Compact8
     //    210 -> 189 (28 rows 199).  Shorter ragged y- and z-lines keep 16 rows
     //    (165 points: 67 against 70 us), longer ones 32.
-    // Fewer lines stay on the LDS-tiled kernel, although 20 rows would be faster
-    // there too (272 Penta10 lines of 131 points 21 -> 11 us): a launch of so
-    // small a box is mostly latency.
+    // Fewer lines stay on the LDS-tiled kernel.  The limit is a cautious one, not
+    // where the gain ends: 272 Penta10 lines of 131 points 21 -> 11 us in 20 rows.
     const bool auto_rows = banded(cls, kind) && !tune.mm && tune.family != 2;
     const bool mid = found && dir != 0 && op->plan.cshort >= 0 && op->plan.MM == 32 && dims[dir] <= 320;
     if (auto_rows && !singular && nlines >= 512 && (!found || mid)) {
@@ -264,7 +263,8 @@ int choose(int cls, int kind, int dir, int bc, const int bc3[3], const int dims[
         const mc3d::OpDev d32 = op->dev;
         found = false;
         for (int mm : {20, 28})
-            if (!found && dims[dir] % mm != 0 && !(mid && mm == 28)) found = plan_with(mm) == MC3D_OK && op->fast;
+            if (!found && dims[dir] % mm != 0 && dims[dir] <= 16 * mm && !(mid && mm == 28))
+                found = plan_with(mm) == MC3D_OK && op->fast;
         if (!found && mid) op->plan = p32, op->dev = d32, op->fast = found = true;
     }
     // few lines that 16-row chunks leave too short a remainder (241 points)
