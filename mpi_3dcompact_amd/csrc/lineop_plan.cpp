@@ -443,6 +443,11 @@ int build_plan(const PlanRequest &rq, Plan &plan, std::string &err) {
     // takes 16- and 32-row tables, so those requests keep its limits).
     const int rem = n - (P - 1) * mm;
     const bool short2 = n % mm != 0 && P >= 3 && rem >= std::max(2 * W, 1);
+    // (32 rows, the last resort: where that shorter chunk does not hold its
+    // interface blocks either, more chunks until it does; 993 points and W = 1:
+    // 33 chunks of 30 rows and one of 3, not 31 of 32 and one of 1)
+    if (mm == 32 && !short2)
+        for (; last < std::max(2 * W, 1) && M > 2 * W; ++P, M = (n + P - 1) / P, last = n - (P - 1) * M) {}
     if (!(short2 && mm % 16 != 0) && (last < std::max(2 * W, 1) || M > mm)) { err = "cannot partition line"; return -1; }
     plan.cshort = -1;
     plan.lshort = 0;

@@ -36,13 +36,14 @@ def test_plan_replay(monkeypatch, n, mm):
 
 @pytest.mark.parametrize("others", [(8, 9), (32, 24)])
 def test_every_length_has_a_kernel(others):
-    """Every operator is accepted on every length from 11 to 992 points, whatever
-    remainder 16- and 32-row chunks leave; 993 = 31 x 32 + 1 has no split that a
-    kernel takes, and a singular operator is refused as one at every length."""
+    """Every operator is accepted on every length from 11 to 4096 points, whatever
+    remainder 16- and 32-row chunks leave, and a singular operator is refused as
+    one at every length."""
     from mpi_3dcompact_amd._lib import Mc3dError
     from mpi_3dcompact_amd.ops import plan_kernel
-    short = (211, 226, 227, 241, 242, 243, 257, 258, 259, 289, 321, 322, 323, 353, 481, 609, 641, 737, 865, 961)
-    for n in [*range(11, 260, 3), *short, 992]:
+    short = (211, 226, 227, 241, 242, 243, 257, 258, 259, 289, 321, 322, 323, 353, 481, 609, 641, 737, 865, 961,
+             993, 994, 995, 1025, 1026, 1057)
+    for n in [*range(11, 260, 3), *short]:
         for d in range(3):
             dims = list(others)
             dims.insert(d, n)
@@ -51,8 +52,8 @@ def test_every_length_has_a_kernel(others):
                     bc3 = [0, 0, 0]
                     bc3[d] = bc
                     assert plan_kernel(cls, kind, d, bc3, dims, 0.1, af).startswith("lineop_")
-    with pytest.raises(Mc3dError, match="cannot partition line"):
-        plan_kernel(1, P.COMPACT8, 1, (0, 0, 0), (32, 993, 24), 1.0, 0.49)
+    for n in (2049, 4033):
+        assert plan_kernel(0, P.PADE6, 1, (1, 1, 1), (32, n, 24)).startswith("lineop_kernel<")
     for n in (64, 257):
         with pytest.raises(Mc3dError, match="zero pivot"):
             plan_kernel(1, P.COMPACT8, 1, (0, 0, 0), (32, n, 24), 1.0, 1.0)
@@ -79,6 +80,32 @@ def test_rules_follow_the_device(cus):
         assert f", {four}, " in rows(2, (48 * cus, 1, n)) and ", 32, " in rows(2, (48 * cus + 1, 1, n))
     for n, lines in ((112, 3 * 64 * cus), (150, 16 * cus), (160, 64 * cus + 1), (256, 64 * cus + 1)):
         assert "_groups<" in rows(0, (n, lines, 1)) and "_groups<" not in rows(0, (n, lines - 1, 1)), n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [993, 1026])
+@pytest.mark.parametrize("d", [0, 1, 2])
+def test_long_short_remainders(n, d):
+    """Lines above 992 points whose remainder over 32 rows is too short, in more
+    chunks of fewer rows, against the oracle at the operators' 1e-12."""
+    import torch
+    from mpi_3dcompact_amd.ops import LineOp
+    dims = [11, 12]
+    dims.insert(d, n)
+    dims = tuple(dims)
+    f = np.random.default_rng(n + d).normal(size=dims[::-1])
+    fin = torch.from_numpy(f).cuda()
+    out = torch.empty_like(fin)
+    for cls, kind, af in OPS:
+        for bc in (P.PERIODIC, P.DIRICHLET):
+            dd = 1.0 / n if bc == P.PERIODIC else 1.0 / (n - 1)
+            bc3 = [0, 0, 0]
+            bc3[d] = bc
+            op = LineOp.deriv(kind, d, bc, dims, dd) if cls == 0 else LineOp.filter(kind, af, d, bc3, dims)
+            print(f"n={n} dir={d} cls={cls} kind={kind} bc={bc} {op.kernel()}", flush=True)
+            want = P.deriv_field(kind, d, bc, f, dd) if cls == 0 else P.filter_field(kind, af, d, bc3, f)
+            op.apply([fin], [out])
+            assert np.max(np.abs(out.cpu().numpy() - want)) <= 1e-12 * np.max(np.abs(want)), (cls, kind, bc)
 
 
 @pytest.mark.gpu
